@@ -18,6 +18,8 @@ FLAGS = [
     "--offload-arch=" + ARCH, "-O3", "-std=c++17", "-fPIC", "-Wall", "-Wno-unused-function",
     # packed FP32 instructions are kept out of the generated code
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
+    # matrix products leave their results in the registers that vector instructions read
+    "-mllvm", "-amdgpu-mfma-vgpr-form=1",
     "-I" + os.path.join(HERE, "..", "include"),
 ]
 

@@ -737,6 +737,12 @@ int frame_ready(pisurf_ctx* c) {
     return PISURF_OK;
 }
 
+// points per hash cell of a level's lattice with per_width points along a node's width
+double lattice_density(const pisurf_ctx* c, int level_depth, int per_width) {
+    const double per_cell = (double)c->g.cell * per_width / (2 * std::ldexp((double)c->root_half, -level_depth));
+    return per_cell * per_cell * per_cell;
+}
+
 // run the three level kernels on `lv` (nodes already in lv.c / depth / id)
 int sweep(pisurf_ctx* c, LevelBuf* L, int32_t* sc_dev, int level_depth) {
     const int prec = prec_of(c);
@@ -849,7 +855,8 @@ int sweep(pisurf_ctx* c, LevelBuf* L, int32_t* sc_dev, int level_depth) {
             int kx = 0;
             hipError_t herr = hipSuccess;
             launch_sample_dedupe_eval(prec, c->g, c->rec_a.p, c->rec_g.p, fc, v, L->child.as<int>(), skv,
-                                      tiles ? c->sd_rent.as<int>() : nullptr, 3 * lb, nrec,
+                                      tiles ? c->sd_rent.as<int>() : nullptr, 3 * lb, lattice_density(c, level_depth, 2),
+                                      nrec,
                                       tiles ? c->sd_entrec.as<int>() : nullptr, nent,
                                       tiles ? c->sd_rechead.as<int>() : nullptr, c->sd_head.as<int>(),
                                       c->sd_hpos.as<int>(), c->sd_rep.as<int>(), c->sd_hlist.as<int>(),
@@ -889,6 +896,7 @@ int sweep(pisurf_ctx* c, LevelBuf* L, int32_t* sc_dev, int level_depth) {
             }
             hipError_t herr = hipSuccess;
             launch_centers_runs(prec, c->g, c->rec_a.p, c->rec_g.p, fc, v, c->cl_list.as<int>(), k,
+                                lattice_density(c, level_depth, 1),
                                 c->sd_key.as<uint64_t>(), c->sd_val.as<int>(), c->sd_key2.as<uint64_t>(),
                                 c->sd_val2.as<int>(), c->sd_cwork.as<int>(), c->tmp.as<int>(), c->samples.p, c->ctr(),
                                 c->trial_ctr(), c->hread(), c->stream, &herr);

@@ -167,9 +167,18 @@ __device__ __forceinline__ float ref_poly6(float d2, float h2, float sigma) {
     return p * sigma;
 }
 
-// squared distance of a candidate offset (one expression shared by every field kernel, so the
-// compiler forms the same operations everywhere)
-template <class R> __device__ __forceinline__ R dist2(R dx, R dy, R dz) { return dx * dx + dy * dy + dz * dz; }
+// a b + c d + e f with the fused operations written out: left to contraction, which product of a sum is fused depends
+// on the code around it, and kernels that sum the same point would round differently
+__device__ __forceinline__ float dot3(float a, float b, float c, float d, float e, float f) {
+#pragma clang fp contract(off)
+    return __builtin_fmaf(e, f, __builtin_fmaf(a, b, c * d));
+}
+__device__ __forceinline__ double dot3(double a, double b, double c, double d, double e, double f) {
+#pragma clang fp contract(off)
+    return __builtin_fma(e, f, __builtin_fma(a, b, c * d));
+}
+// squared distance of a candidate offset
+template <class R> __device__ __forceinline__ R dist2(R dx, R dy, R dz) { return dot3(dx, dx, dy, dy, dz, dz); }
 
 // kernel choice of the field sums: read from FieldConst at run time, or fixed at compile time to
 // the default anisotropic B-spline (use_ani = 1, use_poly6 = 0)
@@ -222,10 +231,10 @@ __device__ __forceinline__ void field_contrib(const FieldConst& fc, R inv_h2, R 
         dz -= R(lo.z);
     }
     if (ani) {
-        const R gx = g0.x * dx + g0.y * dy + g0.z * dz;
-        const R gy = g0.y * dx + g0.w * dy + g1.x * dz;
-        const R gz = g0.z * dx + g1.x * dy + g1.y * dz;
-        const R n2 = gx * gx + gy * gy + gz * gz;
+        const R gx = dot3(g0.x, dx, g0.y, dy, g0.z, dz);
+        const R gy = dot3(g0.y, dx, g0.w, dy, g1.x, dz);
+        const R gz = dot3(g0.z, dx, g1.x, dy, g1.y, dz);
+        const R n2 = dot3(gx, gx, gy, gy, gz, gz);
         if (poly6) {
             const R t = h2 - n2;
             if (!(n2 > h2)) acc.add_unfused(g1.z * (t * t * t));

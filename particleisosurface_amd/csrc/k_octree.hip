@@ -7,6 +7,7 @@
 #include "qef_device.h"
 #include "run_eval.h"
 #include "run_tuner.h"
+#include "wave_eval.h"
 
 #include <cmath>
 #include <type_traits>
@@ -407,6 +408,19 @@ __global__ void __launch_bounds__(T) k_run_centers(GridDev g, Recs<R> rec, Field
     if (threadIdx.x == 0) atomicAdd(&c->field_evals, (unsigned long long)(h1 - h0));
 }
 
+// the same with 64 consecutive centres (in cell order) per wave
+template <class R, bool K, int T, int MODE>
+__global__ void __launch_bounds__(T) k_wave_centers(GridDev g, Recs<R> rec, FieldConst fc, NodeLevel lv,
+                                                    const int* __restrict__ list, SortedKV kv, int n,
+                                                    R* __restrict__ samples, Counters* ctr) {
+    __shared__ WaveLds<WaveField<R, K, false, MODE>> lds[T / kWave];
+    const CenterSrc<R> src{lv, list, kv, samples, R(fc.iso), out_sigma<R, K>(fc)};
+    const int vis = wave_eval<T, R, K, false, MODE>(g, rec, fc, src, n, lds);
+    Counters* c = ctr_stripe(ctr);
+    wave_count(&c->candidates, (unsigned long long)vis);
+    if (threadIdx.x == 0) atomicAdd(&c->field_evals, (unsigned long long)min(T, n - (int)blockIdx.x * T));
+}
+
 // Cell groups of nh points in cell-major order (key[hlist[h]] >> gshift is the cell group of point
 // h; hlist NULL: point h is entry h). cwork: flags | positions | group starts, run starts
 // ((nh + 2) + (nh + 2) + 2 (nh + 2) ints). Returns the number of groups (one read-back; 0 with *err
@@ -680,6 +694,26 @@ __global__ void __launch_bounds__(T) k_run_samples(GridDev g, Recs<R> rec, Field
     if (threadIdx.x == 0) {
         atomicAdd(&c->sample_unique, (unsigned long long)(h1 - h0));
         atomicAdd(&c->run_evals, (unsigned long long)(h1 - h0));
+    }
+}
+
+// the same with 64 consecutive points (in cell order) per wave
+template <class R, bool K, int T, int MODE>
+__global__ void __launch_bounds__(T) k_wave_samples(GridDev g, Recs<R> rec, FieldConst fc, NodeLevel lv,
+                                                    const int* __restrict__ list, SortedKV kv,
+                                                    const int* __restrict__ hlist, int n, R* __restrict__ out,
+                                                    const int* __restrict__ ent, Counters* ctr) {
+    __shared__ WaveLds<WaveField<R, K, false, MODE>> lds[T / kWave];
+    const SampleSrc<R> src{lv, list, kv, hlist, out, R(fc.iso), out_sigma<R, K>(fc), ent};
+    const unsigned long long vis = wave_eval<T, R, K, false, MODE>(g, rec, fc, src, n, lds);
+    Counters* c = ctr_stripe(ctr);
+    wave_count(&c->sample_candidates, vis);
+    wave_count(&c->candidates, vis);
+    wave_count(&c->run_candidates, vis);
+    if (threadIdx.x == 0) {
+        const unsigned long long m = (unsigned long long)min(T, n - (int)blockIdx.x * T);
+        atomicAdd(&c->sample_unique, m);
+        atomicAdd(&c->run_evals, m);
     }
 }
 
@@ -1100,8 +1134,31 @@ static void launch_run_samples(int prec, int T, GridDev g, const void* ra, const
     else m1 ? go(std::integral_constant<int, 128>(), M1()) : go(std::integral_constant<int, 128>(), M0());
 }
 
+// one launch of the sample waves
+static void launch_wave_samples(int prec, int T, GridDev g, const void* ra, const void* rg, FieldConst fc, NodeLevel lv,
+                                const int* list, SortedKV kv, const int* hlist, int nh, void* vals, const int* ent,
+                                Counters* ctr, hipStream_t s) {
+    const unsigned nb = (unsigned)((nh + T - 1) / T);
+    wave_dispatch(T, field_mode(fc), [&](auto tag, auto mode) {
+        constexpr int TT = decltype(tag)::value, M = decltype(mode)::value;
+        if (prec == 2) {
+            Recs<double> r{(const double4*)ra, (const double4*)rg};
+            k_wave_samples<double, false, TT, M><<<nb, TT, 0, s>>>(g, r, fc, lv, list, kv, hlist, nh, (double*)vals, ent,
+                                                                   ctr);
+        } else {
+            Recs<float> r{(const float4*)ra, (const float4*)rg};
+            if (prec == 1)
+                k_wave_samples<float, true, TT, M><<<nb, TT, 0, s>>>(g, r, fc, lv, list, kv, hlist, nh, (float*)vals,
+                                                                     ent, ctr);
+            else
+                k_wave_samples<float, false, TT, M><<<nb, TT, 0, s>>>(g, r, fc, lv, list, kv, hlist, nh, (float*)vals,
+                                                                      ent, ctr);
+        }
+    });
+}
+
 void launch_sample_dedupe_eval(int prec, GridDev g, const void* ra, const void* rg, FieldConst fc, NodeLevel lv,
-                               const int* list, SortedKV kv, const int* ent, int gshift, int64_t nrec,
+                               const int* list, SortedKV kv, const int* ent, int gshift, double density, int64_t nrec,
                                const int* ent_rec, int64_t nent, int* rec_head, int* head, int* hpos, int* rep,
                                int* hlist, int* cwork, int64_t* nheads_out, int64_t* nruns_out, int* kx_out,
                                void* vals, void* samples, int* tmp, Counters* ctr, Counters* trial_ctr, hipEvent_t e0,
@@ -1124,22 +1181,33 @@ void launch_sample_dedupe_eval(int prec, GridDev g, const void* ra, const void* 
         return;
     }
     *nheads_out = nh;
-    const int ng = build_groups(kv, gshift, hlist, nh, cwork, tmp, rd, s, err);
     int* rstart = nullptr;
     int nr = 0;
-    (void)hipEventRecord(e0, s);
-    if (ng > 0) {
-        const RunShape sh = tuned_run_launch(
-            prec, kRunSamples, (double)nh / ng, trial_ctr, s,
-            [&](RunShape c) {
-                nr = build_run_starts(g, kv, gshift, hlist, nh, ng, c.kx, cwork, tmp, &rstart, rd, s, err);
-                return nr > 0;
-            },
+    if (density >= kWaveDensity && nh >= kWaveMin) {
+        (void)hipEventRecord(e0, s);
+        tuned_run_launch(
+            prec, kRunSamples, density, true, trial_ctr, s, [](RunShape) { return true; },
             [&](RunShape c, bool trial) {
-                launch_run_samples(prec, c.T, g, ra, rg, fc, lv, list, kv, hlist, rstart, vals, nr, ent,
-                                   trial ? trial_ctr : ctr, s);
+                launch_wave_samples(prec, c.T, g, ra, rg, fc, lv, list, kv, hlist, nh, vals, ent,
+                                    trial ? trial_ctr : ctr, s);
             });
-        *kx_out = sh.kx;
+        nr = (nh + kWave - 1) / kWave;
+    } else {
+        const int ng = build_groups(kv, gshift, hlist, nh, cwork, tmp, rd, s, err);
+        (void)hipEventRecord(e0, s);
+        if (ng > 0) {
+            const RunShape sh = tuned_run_launch(
+                prec, kRunSamples, (double)nh / ng, false, trial_ctr, s,
+                [&](RunShape c) {
+                    nr = build_run_starts(g, kv, gshift, hlist, nh, ng, c.kx, cwork, tmp, &rstart, rd, s, err);
+                    return nr > 0;
+                },
+                [&](RunShape c, bool trial) {
+                    launch_run_samples(prec, c.T, g, ra, rg, fc, lv, list, kv, hlist, rstart, vals, nr, ent,
+                                       trial ? trial_ctr : ctr, s);
+                });
+            *kx_out = sh.kx;
+        }
     }
     *nruns_out = nr;
     (void)hipEventRecord(e1, s);
@@ -1167,8 +1235,8 @@ void launch_centers(int prec, GridDev g, const void* ra, const void* rg, FieldCo
 }
 
 void launch_centers_runs(int prec, GridDev g, const void* ra, const void* rg, FieldConst fc, NodeLevel lv,
-                         const int* list, int64_t k, uint64_t* key, int* val, uint64_t* key2, int* val2, int* cwork,
-                         int* tmp, void* samples, Counters* ctr, Counters* trial_ctr, HostRead* rd,
+                         const int* list, int64_t k, double density, uint64_t* key, int* val, uint64_t* key2, int* val2,
+                         int* cwork, int* tmp, void* samples, Counters* ctr, Counters* trial_ctr, HostRead* rd,
                          hipStream_t s, hipError_t* err) {
     if (k <= 0) return;
     const uint64_t groups = (uint64_t)(g.n[0] + 2) * (uint64_t)(g.n[1] + 2) * (uint64_t)(g.n[2] + 2);
@@ -1177,6 +1245,31 @@ void launch_centers_runs(int prec, GridDev g, const void* ra, const void* rg, Fi
     const int vbits = pack_vbits(bits, k);
     k_center_keys<<<(unsigned)((k + 255) / 256), 256, 0, s>>>(g, lv, list, k, vbits, key, val);
     const SortedKV kv = radix_sort_entries(key, val, key2, val2, k, bits, vbits, tmp, s);
+    if (density >= kWaveDensity && k >= kWaveMin) {
+        tuned_run_launch(
+            prec, kRunCenters, density, true, trial_ctr, s, [](RunShape) { return true; },
+            [&](RunShape c, bool trial) {
+                Counters* cc = trial ? trial_ctr : ctr;
+                const unsigned nb = (unsigned)((k + c.T - 1) / c.T);
+                wave_dispatch(c.T, field_mode(fc), [&](auto tag, auto mode) {
+                    constexpr int TT = decltype(tag)::value, M = decltype(mode)::value;
+                    if (prec == 2) {
+                        Recs<double> r{(const double4*)ra, (const double4*)rg};
+                        k_wave_centers<double, false, TT, M><<<nb, TT, 0, s>>>(g, r, fc, lv, list, kv, (int)k,
+                                                                               (double*)samples, cc);
+                    } else {
+                        Recs<float> r{(const float4*)ra, (const float4*)rg};
+                        if (prec == 1)
+                            k_wave_centers<float, true, TT, M><<<nb, TT, 0, s>>>(g, r, fc, lv, list, kv, (int)k,
+                                                                                 (float*)samples, cc);
+                        else
+                            k_wave_centers<float, false, TT, M><<<nb, TT, 0, s>>>(g, r, fc, lv, list, kv, (int)k,
+                                                                                  (float*)samples, cc);
+                    }
+                });
+            });
+        return;
+    }
     const int ng = build_groups(kv, 0, nullptr, (int)k, cwork, tmp, rd, s, err);
     if (ng <= 0) return;
     int* rstart = nullptr;
@@ -1206,7 +1299,7 @@ void launch_centers_runs(int prec, GridDev g, const void* ra, const void* rg, Fi
         else m1 ? go(std::integral_constant<int, 128>(), M1()) : go(std::integral_constant<int, 128>(), M0());
     };
     tuned_run_launch(
-        prec, kRunCenters, (double)k / ng, trial_ctr, s,
+        prec, kRunCenters, (double)k / ng, false, trial_ctr, s,
         [&](RunShape c) {
             nr = build_run_starts(g, kv, 0, nullptr, (int)k, ng, c.kx, cwork, tmp, &rstart, rd, s, err);
             return nr > 0;

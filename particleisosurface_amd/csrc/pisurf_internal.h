@@ -186,8 +186,8 @@ void launch_centers(int prec, GridDev g, const void* rec_a, const void* rec_g, F
 // runs of cells; key / val / key2 / val2 hold k entries, cwork 4 (k + 2) ints. The counts of groups
 // and runs are read back through rd; a failed read sets *err (left untouched otherwise).
 void launch_centers_runs(int prec, GridDev g, const void* rec_a, const void* rec_g, FieldConst fc, NodeLevel lv,
-                         const int* list, int64_t k, uint64_t* key, int* val, uint64_t* key2, int* val2, int* cwork,
-                         int* tmp, void* samples, Counters* ctr, Counters* trial_ctr, HostRead* rd,
+                         const int* list, int64_t k, double density, uint64_t* key, int* val, uint64_t* key2,
+                         int* val2, int* cwork, int* tmp, void* samples, Counters* ctr, Counters* trial_ctr, HostRead* rd,
                          hipStream_t s, hipError_t* err);
 // sample deduplication: keys for the nent = 27 * listed entries (hash cell group, then the
 // lattice position modulo 2^lb per axis; the group starts at bit gshift = 3 lb), then (after the
@@ -208,7 +208,7 @@ void launch_sample_tiles(GridDev g, NodeLevel lv, const int* list, int64_t k, co
 // item value v is a record slot, ent[v] its node * 27 + sample, ent_rec the record slot of each of
 // nent entries and rec_head (one int per slot) scratch.
 void launch_sample_dedupe_eval(int prec, GridDev g, const void* rec_a, const void* rec_g, FieldConst fc, NodeLevel lv,
-                               const int* list, SortedKV kv, const int* ent, int gshift, int64_t nrec,
+                               const int* list, SortedKV kv, const int* ent, int gshift, double density, int64_t nrec,
                                const int* ent_rec, int64_t nent, int* rec_head, int* head, int* hpos, int* rep,
                                int* hlist, int* cwork, int64_t* nheads_out, int64_t* nruns_out, int* kx_out,
                                void* vals, void* samples, int* tmp, Counters* ctr, Counters* trial_ctr, hipEvent_t e0,

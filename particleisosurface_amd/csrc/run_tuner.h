@@ -22,9 +22,21 @@
 namespace pisurf {
 
 struct RunShape {
-    int T;   // threads per workgroup (128 or 256)
-    int kx;  // cells per run
+    int T;   // threads per workgroup
+    int kx;  // cells per run, or 0: 64 consecutive points per wave (wave_eval.h)
 };
+
+// Points of a lattice with at least kWaveDensity points per hash cell, and at least kWaveMin of them, go 64 to a
+// wave (wave_eval.h) and no runs are built. The octree's levels hold 64 (deepest sampled, leaf centres), 8 and 1
+// points per cell, level by level upwards. At 64 and 8 a wave's points share a few cells, so one test of all of
+// them against the union of their windows beats each thread testing its own window: crown splash, 4 M
+// particles, compensated FP32, 11.9 M + 2.4 M points: 1.65 ms against 2.05 ms as runs, centres 0.46 against
+// 0.57 ms. At 1 a wave spans five row pieces and tests 18 candidates for each one in a point's
+// window: 0.70 ms against 0.52 ms for D_min's 1.05 M points. A launch of few points lasts as long as its
+// slowest wave, and a wave of 64 points in several rows is slower than a small run: a 14 k-particle frame's
+// 120 k points took 128 us against 53 us; above 2^18 points both kinds fill the chip.
+constexpr double kWaveDensity = 4.0;
+constexpr int64_t kWaveMin = 1 << 18;
 
 // kx p is about 90 % of T (a run may hold more points than the average) and the block size that
 // keeps more of its threads busy wins; a cell of more than T points is taken in several passes
@@ -46,7 +58,8 @@ inline RunShape run_shape_guess(double p) {
 // the heuristic shape, then for each block size a ladder of cells per run from a quarter to twice
 // its heuristic count (the mean p counts empty cells too, so occupied cells can hold several times
 // p points)
-inline std::vector<RunShape> run_shape_candidates(double p) {
+inline std::vector<RunShape> run_shape_candidates(double p, bool wave) {
+    if (wave) return {RunShape{256, 0}, RunShape{128, 0}, RunShape{64, 0}};
     std::vector<RunShape> c;
     auto add = [&](RunShape s) {
         s.kx = std::max(1, std::min(128, s.kx));
@@ -109,17 +122,18 @@ class RunTuner {
 // timed (trial = true: count into the scratch block); returns the shape whose launch's results
 // stand (the last one run). `prepare` builds the runs of a shape (it may read counts back) and
 // returns false to skip the launch.
+// wave: 64 points per wave (p is then the density that names the bucket) instead of runs of cells.
 template <class Prepare, class Launch>
-RunShape tuned_run_launch(int prec, int kind, double p, void* scratch_ctr, hipStream_t s, Prepare&& prepare,
+RunShape tuned_run_launch(int prec, int kind, double p, bool wave, void* scratch_ctr, hipStream_t s, Prepare&& prepare,
                           Launch&& launch) {
     RunTuner& tu = RunTuner::get();
-    const long k = RunTuner::key(prec, kind, RunTuner::bucket(p));
-    RunShape sh = run_shape_guess(p);
+    const long k = RunTuner::key(prec, wave ? kind + 4 : kind, RunTuner::bucket(p));
+    RunShape sh = wave ? RunShape{256, 0} : run_shape_guess(p);
     if (!tu.enabled() || tu.lookup(k, &sh) || !scratch_ctr) {
         if (prepare(sh)) launch(sh, false);
         return sh;
     }
-    const std::vector<RunShape> cand = run_shape_candidates(p);
+    const std::vector<RunShape> cand = run_shape_candidates(p, wave);
     hipEvent_t e0 = nullptr, e1 = nullptr;
     if (hipEventCreate(&e0) != hipSuccess || hipEventCreate(&e1) != hipSuccess) {
         if (e0) (void)hipEventDestroy(e0);
