@@ -40,3 +40,22 @@ def test_wave_sums_equal_per_point_sums(frame, prec, ani, poly6):
         assert np.array_equal(na[key], nb[key]), key
     assert np.array_equal(ma[0], mb[0]) and np.array_equal(ma[1], mb[1])
     assert sa["field_evals"] == sb["field_evals"]
+
+
+@pytest.mark.parametrize("nq", [1, 3, 4, 5, 257])
+def test_neighbor_lists_of_few_queries(nq):
+    """One wave per query: counts that leave waves of a workgroup without one, queries in a dense cluster
+    (lists of several hundred ids), alone in their cells and off the grid, against the reference order."""
+    xyz, r = synth.random_cloud(900, r=0.01, extent=0.1)
+    far = np.array([[0.5, 0.5, 0.5], [0.5, 0.62, 0.5]], np.float32)
+    xyz = np.concatenate([xyz, far])
+    q = np.concatenate([far, xyz[:300], [[9.0, 0.0, 0.0]]]).astype(np.float32)[-nq:]
+    ctx = gpu_context(xyz, r)
+    ctx.hashgrid_build()
+    off, ids = ctx.neighbors(q)
+    from oracle.pyoracle import Oracle
+    o = Oracle(xyz, r)
+    o.hashgrid_build()
+    off2, ids2 = o.neighbors(q)
+    assert np.array_equal(off, off2) and np.array_equal(ids, ids2[:off2[-1]])
+    ctx.close()
