@@ -1546,6 +1546,29 @@ int do_extract_device(pisurf_ctx* c) {
     return PISURF_OK;
 }
 
+// field (and gradient) at n points in device memory; records and constants ready
+int eval_points(pisurf_ctx* c, const float* q, int64_t n, double* f, double* grad) {
+    bool sorted = eval_points_sorts(n, c->n);
+    if (sorted) {
+        // without room for the sort (16 B a point and its tables) the points are taken as they come
+        const int64_t need = radix_tmp_ints(n) + 64;
+        sorted = c->sd_key.ensure(n * 8) == hipSuccess && c->sd_key2.ensure(n * 8) == hipSuccess &&
+                 c->sd_val.ensure(n * 4) == hipSuccess && c->sd_val2.ensure(n * 4) == hipSuccess;
+        if (sorted && (size_t)need * 4 > c->tmp.cap) {
+            HIPCHK(c, c->wait());
+            sorted = c->tmp.ensure(need * 4) == hipSuccess;
+        }
+        if (!sorted) (void)hipGetLastError();
+    }
+    if (sorted)
+        launch_eval_points_sorted(prec_of(c), c->g, c->rec_a.p, c->rec_g.p, field_const(c), q, n, f, grad,
+                                  c->sd_key.as<uint64_t>(), c->sd_val.as<int>(), c->sd_key2.as<uint64_t>(),
+                                  c->sd_val2.as<int>(), c->tmp.as<int>(), c->ctr(), c->stream);
+    else
+        launch_eval_points(prec_of(c), c->g, c->rec_a.p, c->rec_g.p, field_const(c), q, n, f, grad, c->ctr(), c->stream);
+    return PISURF_OK;
+}
+
 int do_extract(pisurf_ctx* c);
 
 int do_extract_host(pisurf_ctx* c);
@@ -2374,8 +2397,8 @@ int pisurf_eval_points(pisurf_ctx* c, const float* q, int64_t n, double* f, doub
     HIPCHK(c, c->out1.ensure(n * 8));
     if (grad) HIPCHK(c, c->out2.ensure(n * 24));
     HIPCHK(c, hipMemcpyAsync(c->q.p, q, n * 12, hipMemcpyHostToDevice, c->stream));
-    launch_eval_points(prec_of(c), c->g, c->rec_a.p, c->rec_g.p, field_const(c), c->q.as<float>(), n,
-                       c->out1.as<double>(), grad ? c->out2.as<double>() : nullptr, c->ctr(), c->stream);
+    rc = eval_points(c, c->q.as<float>(), n, c->out1.as<double>(), grad ? c->out2.as<double>() : nullptr);
+    if (rc) return rc;
     HIPCHK(c, hipGetLastError());
     HIPCHK(c, hipMemcpyAsync(f, c->out1.p, n * 8, hipMemcpyDeviceToHost, c->stream));
     if (grad) HIPCHK(c, hipMemcpyAsync(grad, c->out2.p, n * 24, hipMemcpyDeviceToHost, c->stream));

@@ -80,6 +80,13 @@ template <class R> __device__ __forceinline__ R dsqrt(R x);
 template <> __device__ __forceinline__ float dsqrt<float>(float x) { return __builtin_amdgcn_sqrtf(x); }
 template <> __device__ __forceinline__ double dsqrt<double>(double x) { return sqrt(x); }
 
+// LDS written by some lanes of the wave is read by others
+__device__ __forceinline__ void wave_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // inclusive prefix sum over the 64 lanes of a wave
 __device__ __forceinline__ int wave_incl_scan(int v, int lane) {
 #pragma unroll
@@ -176,6 +183,13 @@ __device__ __forceinline__ float dot3(float a, float b, float c, float d, float 
 __device__ __forceinline__ double dot3(double a, double b, double c, double d, double e, double f) {
 #pragma clang fp contract(off)
     return __builtin_fma(e, f, __builtin_fma(a, b, c * d));
+}
+// iso - sigma sum, fused alike everywhere
+__device__ __forceinline__ float field_value(float iso, float sigma, float sum) {
+    return __builtin_fmaf(-sigma, sum, iso);
+}
+__device__ __forceinline__ double field_value(double iso, double sigma, double sum) {
+    return __builtin_fma(-sigma, sum, iso);
 }
 // squared distance of a candidate offset
 template <class R> __device__ __forceinline__ R dist2(R dx, R dy, R dz) { return dot3(dx, dx, dy, dy, dz, dz); }

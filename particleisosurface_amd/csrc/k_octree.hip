@@ -189,17 +189,6 @@ __global__ void k_sample_flag(TreeParams tp, NodeLevel lv, int* __restrict__ fla
 // evaluation; only copies with bitwise-identical float coordinates are merged, so every value is
 // exactly what the node's own evaluation would produce.
 
-// Hash cell group of a point for the run evaluation: its cell (CalcXYZIdx) in the grid
-// extended by one cell on every side; points farther out have an empty 27-cell window and share
-// the last group. Points of one group have the same candidate list in the same order.
-__device__ __forceinline__ uint64_t cell_group(const GridDev& g, float x, float y, float z) {
-    int ix, iy, iz;
-    cell_of(g, x, y, z, ix, iy, iz);
-    const uint64_t ex = g.n[0] + 2, ey = g.n[1] + 2, ez = g.n[2] + 2;
-    if (ix < -1 || ix > g.n[0] || iy < -1 || iy > g.n[1] || iz < -1 || iz > g.n[2]) return ex * ey * ez;
-    return ((uint64_t)(iz + 1) * ey + (uint64_t)(iy + 1)) * ex + (uint64_t)(ix + 1);
-}
-
 // key of sample entry t: the point's cell group, then its lattice position modulo 2^lb per axis
 // (lb bits: enough for the lattice steps a cell spans). Equal points have equal keys; distinct
 // points that share one are told apart by the heads pass, which compares coordinates.
@@ -390,7 +379,7 @@ template <class R> struct CenterSrc {
         p[2] = c.z;
     }
     __device__ __forceinline__ void store(int h, R sum, const R*) const {
-        samples[(int64_t)list[kv.val(h)] * 27 + 13] = iso - sigma * sum;
+        samples[(int64_t)list[kv.val(h)] * 27 + 13] = field_value(iso, sigma, sum);
     }
 };
 
@@ -674,7 +663,7 @@ template <class R> struct SampleSrc {
     R iso, sigma;
     const int* ent = nullptr;  // sorted item -> node * 27 + sample (nullptr: the items are the list's entries)
     __device__ __forceinline__ void point(int h, float p[3]) const { item_point(lv, list, ent, kv.val(hlist[h]), p); }
-    __device__ __forceinline__ void store(int h, R sum, const R*) const { out[h] = iso - sigma * sum; }
+    __device__ __forceinline__ void store(int h, R sum, const R*) const { out[h] = field_value(iso, sigma, sum); }
 };
 
 template <class R, bool K, int T, int MODE>
@@ -749,7 +738,7 @@ __global__ void __launch_bounds__(256) k_centers(GridDev g, Recs<R> rec, FieldCo
         const float4 c = lv.c[node];
         R sum, gr[3];
         vis = field_sum<R, K, false>(g, rec, fc, c.x, c.y, c.z, R(c.x), R(c.y), R(c.z), sum, gr);
-        samples[node * 27 + 13] = R(fc.iso) - out_sigma<R, K>(fc) * sum;
+        samples[node * 27 + 13] = field_value(R(fc.iso), out_sigma<R, K>(fc), sum);
         did = true;
     }
     wave_count(&ctr_stripe(ctr)->field_evals, did ? 1ull : 0ull);
@@ -778,7 +767,7 @@ __global__ void __launch_bounds__(256) k_samples(GridDev g, Recs<R> rec, FieldCo
         sample_point(lv.c[node], s, p);
         R sum, gr[3];
         vis = field_sum<R, K, false>(g, rec, fc, p[0], p[1], p[2], R(p[0]), R(p[1]), R(p[2]), sum, gr);
-        samples[node * 27 + s] = R(fc.iso) - out_sigma<R, K>(fc) * sum;
+        samples[node * 27 + s] = field_value(R(fc.iso), out_sigma<R, K>(fc), sum);
         did = true;
     }
     wave_count(&ctr_stripe(ctr)->field_evals, did ? 1ull : 0ull);
@@ -844,7 +833,7 @@ __global__ void __launch_bounds__(256) k_classify(GridDev g, Recs<R> rec, FieldC
                         vis += field_sum<R, K, false, kModeAny, true>(g, rec, fc, c.x, c.y, c.z, R(c.x), R(c.y),
                                                                      R(c.z), sum, g3);
                         evals++;
-                        fval = R(fc.iso) - out_sigma<R, K>(fc) * sum;
+                        fval = field_value(R(fc.iso), out_sigma<R, K>(fc), sum);
                     }
                 }
             }
@@ -876,7 +865,7 @@ __global__ void __launch_bounds__(256) k_qef_values(GridDev g, Recs<R> rec, Fiel
         R sum, g3[3];
         vis = field_sum<R, K, false, kModeAny, true>(g, rec, fc, float(vx), float(vy), float(vz), vx, vy, vz, sum, g3);
         evals = 1;
-        const R fval = nd.w == 0.0 ? R(0) : R(fc.iso) - out_sigma<R, K>(fc) * sum;
+        const R fval = nd.w == 0.0 ? R(0) : field_value(R(fc.iso), out_sigma<R, K>(fc), sum);
         lv.node[node].w = double(fval);
     }
     wave_count(&ctr_stripe(ctr)->field_evals, evals);
@@ -994,9 +983,7 @@ void launch_sample_scatter(const int* list, SortedKV kv, const int* rep, const i
 
 SortedKV launch_center_keys_sorted(GridDev g, NodeLevel lv, const int* list, int64_t k, uint64_t* key, int* val,
                                    uint64_t* key2, int* val2, int* tmp, hipStream_t s) {
-    const uint64_t groups = (uint64_t)(g.n[0] + 2) * (uint64_t)(g.n[1] + 2) * (uint64_t)(g.n[2] + 2);
-    int bits = 1;
-    while (bits < 55 && ((uint64_t)1 << bits) <= groups) bits++;
+    const int bits = cell_group_bits(g);
     const int vbits = pack_vbits(bits, k);
     if (k <= 0) return SortedKV{key, val, vbits};
     k_center_keys<<<(unsigned)((k + 255) / 256), 256, 0, s>>>(g, lv, list, k, vbits, key, val);
@@ -1239,9 +1226,7 @@ void launch_centers_runs(int prec, GridDev g, const void* ra, const void* rg, Fi
                          int* cwork, int* tmp, void* samples, Counters* ctr, Counters* trial_ctr, HostRead* rd,
                          hipStream_t s, hipError_t* err) {
     if (k <= 0) return;
-    const uint64_t groups = (uint64_t)(g.n[0] + 2) * (uint64_t)(g.n[1] + 2) * (uint64_t)(g.n[2] + 2);
-    int bits = 1;
-    while (bits < 55 && ((uint64_t)1 << bits) <= groups) bits++;
+    const int bits = cell_group_bits(g);
     const int vbits = pack_vbits(bits, k);
     k_center_keys<<<(unsigned)((k + 255) / 256), 256, 0, s>>>(g, lv, list, k, vbits, key, val);
     const SortedKV kv = radix_sort_entries(key, val, key2, val2, k, bits, vbits, tmp, s);

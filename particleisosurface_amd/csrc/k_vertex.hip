@@ -107,7 +107,7 @@ __global__ void __launch_bounds__(64) k_qef(GridDev g, Recs<R> rec, FieldConst f
         }
         R sum, g3[3];
         vis = field_sum<R, K, false>(g, rec, fc, float(vx), float(vy), float(vz), vx, vy, vz, sum, g3);
-        R fv = R(fc.iso) - out_sigma<R, K>(fc) * sum;
+        R fv = field_value(R(fc.iso), out_sigma<R, K>(fc), sum);
         if (err / R(__fmul_rn(2.0f, c.w)) < R(0.0001)) fv = R(0);
         out[i] = make_double4(double(vx), double(vy), double(vz), double(fv));
     }

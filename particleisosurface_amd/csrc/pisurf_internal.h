@@ -130,6 +130,12 @@ __device__ __forceinline__ void wave_count(unsigned long long* ctr, unsigned lon
 }
 void launch_eval_points(int prec, GridDev g, const void* rec_a, const void* rec_g, FieldConst fc, const float* q,
                         int64_t n, double* f, double* grad, Counters* ctr, hipStream_t s);
+// the same for many points, sorted by hash cell first (eval_points_sorts says when); key / val / key2 / val2
+// hold n entries, tmp radix_tmp_ints(n) ints
+bool eval_points_sorts(int64_t n, int64_t particles);
+void launch_eval_points_sorted(int prec, GridDev g, const void* rec_a, const void* rec_g, FieldConst fc, const float* q,
+                               int64_t n, double* f, double* grad, uint64_t* key, int* val, uint64_t* key2, int* val2,
+                               int* tmp, Counters* ctr, hipStream_t s);
 // trial_ctr: counter block for the timed trial launches of shape tuning (their counts are not kept)
 void launch_normals(int prec, GridDev g, const void* rec_a, const void* rec_g, FieldConst fc, const float4* spos,
                     int64_t n, int64_t n_invalid, float4* nrm, Counters* ctr, Counters* trial_ctr, hipStream_t s);

@@ -209,12 +209,31 @@ __device__ __forceinline__ unsigned long long run_eval(const GridDev& g, const R
     return run_visit<T>(g, pol, h0, h1, lds);
 }
 
+// Hash cell group of a point for the run evaluation: its cell (CalcXYZIdx) in the grid
+// extended by one cell on every side; points farther out have an empty 27-cell window and share
+// the last group. Points of one group have the same candidate list in the same order.
+__device__ __forceinline__ uint64_t cell_group(const GridDev& g, float x, float y, float z) {
+    int ix, iy, iz;
+    cell_of(g, x, y, z, ix, iy, iz);
+    const uint64_t ex = g.n[0] + 2, ey = g.n[1] + 2, ez = g.n[2] + 2;
+    if (ix < -1 || ix > g.n[0] || iy < -1 || iy > g.n[1] || iz < -1 || iz > g.n[2]) return ex * ey * ez;
+    return ((uint64_t)(iz + 1) * ey + (uint64_t)(iy + 1)) * ex + (uint64_t)(ix + 1);
+}
+
 // run id of a hash cell (extended by one cell on every side): its (y, z) row and x / kx
 __device__ __forceinline__ uint64_t run_of_cell(const GridDev& g, int ix, int iy, int iz, int kx) {
     const uint64_t ex = g.n[0] + 2, ey = g.n[1] + 2, ez = g.n[2] + 2;
     const uint64_t per_row = (ex + kx - 1) / kx;
     if (ix < -1 || ix > g.n[0] || iy < -1 || iy > g.n[1] || iz < -1 || iz > g.n[2]) return ey * ez * per_row;
     return ((uint64_t)(iz + 1) * ey + (uint64_t)(iy + 1)) * per_row + (uint64_t)(ix + 1) / kx;
+}
+
+// bits of the cell groups' keys
+inline int cell_group_bits(const GridDev& g) {
+    const uint64_t groups = (uint64_t)(g.n[0] + 2) * (uint64_t)(g.n[1] + 2) * (uint64_t)(g.n[2] + 2);
+    int bits = 1;
+    while (bits < 55 && ((uint64_t)1 << bits) <= groups) bits++;
+    return bits;
 }
 
 // particle runs: block b covers the particles of cells [x0, x0 + kx) of one grid row (contiguous

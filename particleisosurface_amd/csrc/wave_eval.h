@@ -57,13 +57,6 @@ template <class Pol> struct WaveLds {
     int raw[9 * (kWaveCells + 3)];      // sorted position of cell boundary x0 - 1 + i of row r at 9 i + r
 };
 
-// LDS written by some lanes of the wave is read by others
-__device__ __forceinline__ void wave_sync() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 // after: r[i] of lane group g (16 lanes each) = the former r[g] of lane group i
 __device__ __forceinline__ void wave_transpose4(unsigned r[4]) {
     auto s32 = [](unsigned& a, unsigned& b) {

@@ -59,3 +59,51 @@ def test_neighbor_lists_of_few_queries(nq):
     off2, ids2 = o.neighbors(q)
     assert np.array_equal(off, off2) and np.array_equal(ids, ids2[:off2[-1]])
     ctx.close()
+
+
+@pytest.mark.parametrize("prec", [capi.FP32, capi.FP32_KAHAN, capi.FP64])
+@pytest.mark.parametrize("grad", [False, True])
+def test_many_points_equal_few_points(frame, prec, grad):
+    """2^18 points or more are sorted and summed 64 to a wave, fewer a wave per point (one point per
+    wave up to 4096 of them, several above): the same values bit for bit, whatever the remainders, in
+    the dense cluster (several hundred passing candidates per point), off the grid and for a NaN."""
+    xyz, r = frame
+    s = synth.Stream(17)
+    n = (1 << 18) + 3
+    pick = (s.uniform(n) * len(xyz)).astype(np.int64)
+    q = (xyz[pick] + s.uniform(3 * n, -3 * r, 3 * r).reshape(-1, 3)).astype(np.float32)
+    q[-400:] = xyz[-400:]
+    q[7] = [5.0, 0.1, 0.1]
+    q[11] = [np.nan, 0.1, 0.1]
+    ctx = gpu_context(xyz, r, precision=prec)
+    whole = ctx.eval_points(q, grad=grad)
+    for a, b in ((0, 13), (13, 4000), (4000, 4000 + 4097), (n - 20003, n)):
+        part = ctx.eval_points(q[a:b], grad=grad)
+        if grad:
+            assert np.array_equal(whole[0][a:b], part[0]) and np.array_equal(whole[1][a:b], part[1]), (a, b)
+        else:
+            assert np.array_equal(whole[a:b], part), (a, b)
+    ctx.close()
+
+
+@pytest.mark.parametrize("prec", [capi.FP32, capi.FP64])
+def test_points_match_oracle(prec):
+    """Points a wave each against the oracle, with single candidates, empty windows and more than 64
+    passing candidates (a cloud of 60 particles per cell)."""
+    from oracle.pyoracle import Oracle
+    xyz, r = synth.random_cloud(4000, r=0.01, extent=0.16)
+    xyz = np.concatenate([xyz, np.array([[0.5, 0.5, 0.5]], np.float32)])
+    q = np.concatenate([xyz[::9], xyz[-1:], xyz[:50] + np.float32(0.2)]).astype(np.float32)
+    ctx = gpu_context(xyz, r, precision=prec)
+    f, g = ctx.eval_points(q, grad=True)
+    o = Oracle(xyz, r, fp64=prec == capi.FP64)
+    o.hashgrid_build()
+    o.set_aniso(*ctx.aniso())
+    iso = o.iso_constants()[1]
+    f2, g2 = o.eval_points(q, grad=True)
+    # same records, same order: FP32 rounds each term as the oracle does (libm's pow may differ by an
+    # ulp per term), FP64 differs by contraction, about 1e-15 per term
+    tol = 2e-6 if prec == capi.FP32 else 1e-13
+    assert np.max(np.abs(f - f2)) <= tol * np.max(np.abs(iso - f2) + iso)
+    assert np.max(np.abs(g - g2)) <= tol * np.max(np.abs(g2))
+    ctx.close()
