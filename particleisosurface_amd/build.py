@@ -11,7 +11,8 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 OBJ = os.path.join(HERE, "_obj")
 LIB = os.path.join(HERE, "libpisurf.so")
-SOURCES = ["k_grid.hip", "k_aniso.hip", "k_field.hip", "k_octree.hip", "k_vertex.hip", "k_extract.hip", "capi.cpp"]
+SOURCES = ["k_grid.hip", "k_aniso.hip", "k_field.hip", "k_octree.hip", "k_vertex.hip", "k_extract.hip", "host_io.hip",
+           "capi.cpp"]
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 ARCH = os.environ.get("PISURF_ARCH", "gfx950")
 FLAGS = [
