@@ -812,71 +812,83 @@ int sweep(pisurf_ctx* c, LevelBuf* L, int32_t* sc_dev, int level_depth) {
         const int64_t nent = (int64_t)k * 27;
         if (nent >= INT32_MAX) return c->fail(PISURF_E_UNSUPPORTED, "octree level has too many sample points");
         if (nent > 0) {
-            // entries merged per tile of nodes first (fewer keys to sort)
-            const bool tiles = L->n * 27 < INT32_MAX;
-            HIPCHK(c, c->sd_key.ensure(nent * 8));
-            HIPCHK(c, c->sd_key2.ensure(nent * 8));
-            HIPCHK(c, c->sd_val.ensure(nent * 4));
-            HIPCHK(c, c->sd_val2.ensure(nent * 4));
-            if (tiles) {
-                HIPCHK(c, c->sd_entrec.ensure(nent * 4));
-                HIPCHK(c, c->sd_rent.ensure(nent * 4));
-                HIPCHK(c, c->sd_rechead.ensure(nent * 4));
-                HIPCHK(c, c->sd_nrec.ensure(4));
-            }
-            HIPCHK(c, c->sd_head.ensure((2 * ((nent + 255) / 256) + 2) * 4));
-            HIPCHK(c, c->sd_hpos.ensure((nent + 1) * 4));
-            HIPCHK(c, c->sd_rep.ensure(nent * 4));
-            HIPCHK(c, c->sd_hlist.ensure(nent * 4));
-            HIPCHK(c, c->sd_vals.ensure(nent * rsz));
-            HIPCHK(c, c->sd_cwork.ensure(4 * (nent + 2) * 4));
-            const int64_t need = std::max(radix_tmp_ints(nent), scan_tmp_ints(nent + 1)) + 64;
-            if ((size_t)need * 4 > c->tmp.cap) {
-                // kernels queued before the count read may still use the workspace
-                HIPCHK(c, c->wait());
-                HIPCHK(c, c->tmp.ensure(need * 4));
-            }
-            const float origin[3] = {c->root_c[0] - c->root_half, c->root_c[1] - c->root_half,
-                                     c->root_c[2] - c->root_half};
-            // distinct points grouped by hash cell (cell-major keys), evaluated in runs of cells
-            const uint64_t groups = (uint64_t)(c->g.n[0] + 2) * (uint64_t)(c->g.n[1] + 2) * (uint64_t)(c->g.n[2] + 2);
-            // three lattice bits per axis: fewer would save a sort pass at the coarser levels but
-            // lengthen the runs of equal keys (shared cells, and the points outside the grid, which
-            // form one group), which costs the heads pass more than the sort gains
-            const int lb = 3;
-            const int kbits = std::min(64, bits_for((int64_t)groups + 1) + 3 * lb);
-            int64_t nrec = nent;
-            const int vbits = pack_vbits(kbits, nent);
-            if (tiles) {
-                launch_sample_tiles(c->g, v, L->child.as<int>(), k, origin, lb, vbits, c->sd_nrec.as<int>(),
-                                    c->sd_entrec.as<int>(), c->sd_key.as<uint64_t>(), c->sd_val.as<int>(),
-                                    c->sd_rent.as<int>(), c->stream);
-                int nr = 0;
-                HIPCHK(c, c->read(&nr, c->sd_nrec.as<int>(), 4));
-                nrec = nr;
-            } else {
-                launch_sample_dedupe_keys(c->g, v, L->child.as<int>(), nent, origin, lb, vbits,
-                                          c->sd_key.as<uint64_t>(), c->sd_val.as<int>(), c->stream);
-            }
-            const SortedKV skv = radix_sort_entries(c->sd_key.as<uint64_t>(), c->sd_val.as<int>(),
-                                                    c->sd_key2.as<uint64_t>(), c->sd_val2.as<int>(), nrec, kbits,
-                                                    vbits, c->tmp.as<int>(), c->stream);
             hipEvent_t e0, e1;
             size_t eslot = 0;
-            HIPCHK(c, c->event_pair(e0, e1, &eslot));
             int64_t nheads = 0, nruns = 0;
-            int kx = 0;
-            hipError_t herr = hipSuccess;
-            launch_sample_dedupe_eval(prec, c->g, c->rec_a.p, c->rec_g.p, fc, v, L->child.as<int>(), skv,
-                                      tiles ? c->sd_rent.as<int>() : nullptr, 3 * lb, lattice_density(c, level_depth, 2),
-                                      nrec,
-                                      tiles ? c->sd_entrec.as<int>() : nullptr, nent,
-                                      tiles ? c->sd_rechead.as<int>() : nullptr, c->sd_head.as<int>(),
-                                      c->sd_hpos.as<int>(), c->sd_rep.as<int>(), c->sd_hlist.as<int>(),
-                                      c->sd_cwork.as<int>(), &nheads, &nruns, &kx, c->sd_vals.p, c->samples.p,
-                                      c->tmp.as<int>(), c->ctr(), c->trial_ctr(), e0, e1, c->hread(), c->stream,
-                                      &herr);
-            HIPCHK(c, herr);
+            // entries merged per tile of nodes first
+            const bool tiles = L->n * 27 < INT32_MAX;
+            const double density = lattice_density(c, level_depth, 2);
+            if (tiles && samples_by_tile(k, density)) {
+                HIPCHK(c, c->sd_nrec.ensure(4));
+                HIPCHK(c, c->sd_entrec.ensure(nent * 4));
+                HIPCHK(c, c->sd_rent.ensure(tile_record_bound(k) * 4));
+                HIPCHK(c, c->sd_vals.ensure(tile_record_bound(k) * rsz));
+                HIPCHK(c, c->event_pair(e0, e1, &eslot));
+                launch_samples_by_tile(prec, c->g, c->rec_a.p, c->rec_g.p, fc, v, L->child.as<int>(), k, density,
+                                       c->sd_nrec.as<int>(), c->sd_entrec.as<int>(), c->sd_rent.as<int>(),
+                                       c->sd_vals.p, c->samples.p, c->ctr(), c->trial_ctr(), e0, e1, c->stream);
+                nruns = 1;
+            } else {
+                HIPCHK(c, c->sd_key.ensure(nent * 8));
+                HIPCHK(c, c->sd_key2.ensure(nent * 8));
+                HIPCHK(c, c->sd_val.ensure(nent * 4));
+                HIPCHK(c, c->sd_val2.ensure(nent * 4));
+                if (tiles) {
+                    HIPCHK(c, c->sd_entrec.ensure(nent * 4));
+                    HIPCHK(c, c->sd_rent.ensure(nent * 4));
+                    HIPCHK(c, c->sd_rechead.ensure(nent * 4));
+                    HIPCHK(c, c->sd_nrec.ensure(4));
+                }
+                HIPCHK(c, c->sd_head.ensure((2 * ((nent + 255) / 256) + 2) * 4));
+                HIPCHK(c, c->sd_hpos.ensure((nent + 1) * 4));
+                HIPCHK(c, c->sd_rep.ensure(nent * 4));
+                HIPCHK(c, c->sd_hlist.ensure(nent * 4));
+                HIPCHK(c, c->sd_vals.ensure(nent * rsz));
+                HIPCHK(c, c->sd_cwork.ensure(4 * (nent + 2) * 4));
+                const int64_t need = std::max(radix_tmp_ints(nent), scan_tmp_ints(nent + 1)) + 64;
+                if ((size_t)need * 4 > c->tmp.cap) {
+                    // kernels queued before the count read may still use the workspace
+                    HIPCHK(c, c->wait());
+                    HIPCHK(c, c->tmp.ensure(need * 4));
+                }
+                const float origin[3] = {c->root_c[0] - c->root_half, c->root_c[1] - c->root_half,
+                                         c->root_c[2] - c->root_half};
+                // distinct points grouped by hash cell (cell-major keys), evaluated in runs of cells
+                const uint64_t groups = (uint64_t)(c->g.n[0] + 2) * (uint64_t)(c->g.n[1] + 2) * (uint64_t)(c->g.n[2] + 2);
+                // three lattice bits per axis: fewer would save a sort pass at the coarser levels but
+                // lengthen the runs of equal keys (shared cells, and the points outside the grid, which
+                // form one group), which costs the heads pass more than the sort gains
+                const int lb = 3;
+                const int kbits = std::min(64, bits_for((int64_t)groups + 1) + 3 * lb);
+                int64_t nrec = nent;
+                const int vbits = pack_vbits(kbits, nent);
+                if (tiles) {
+                    launch_sample_tiles(c->g, v, L->child.as<int>(), k, origin, lb, vbits, c->sd_nrec.as<int>(),
+                                        c->sd_entrec.as<int>(), c->sd_key.as<uint64_t>(), c->sd_val.as<int>(),
+                                        c->sd_rent.as<int>(), c->stream);
+                    int nr = 0;
+                    HIPCHK(c, c->read(&nr, c->sd_nrec.as<int>(), 4));
+                    nrec = nr;
+                } else {
+                    launch_sample_dedupe_keys(c->g, v, L->child.as<int>(), nent, origin, lb, vbits,
+                                              c->sd_key.as<uint64_t>(), c->sd_val.as<int>(), c->stream);
+                }
+                const SortedKV skv = radix_sort_entries(c->sd_key.as<uint64_t>(), c->sd_val.as<int>(),
+                                                        c->sd_key2.as<uint64_t>(), c->sd_val2.as<int>(), nrec, kbits,
+                                                        vbits, c->tmp.as<int>(), c->stream);
+                HIPCHK(c, c->event_pair(e0, e1, &eslot));
+                int kx = 0;
+                hipError_t herr = hipSuccess;
+                launch_sample_dedupe_eval(prec, c->g, c->rec_a.p, c->rec_g.p, fc, v, L->child.as<int>(), skv,
+                                          tiles ? c->sd_rent.as<int>() : nullptr, 3 * lb, nrec,
+                                          tiles ? c->sd_entrec.as<int>() : nullptr, nent,
+                                          tiles ? c->sd_rechead.as<int>() : nullptr, c->sd_head.as<int>(),
+                                          c->sd_hpos.as<int>(), c->sd_rep.as<int>(), c->sd_hlist.as<int>(),
+                                          c->sd_cwork.as<int>(), &nheads, &nruns, &kx, c->sd_vals.p, c->samples.p,
+                                          c->tmp.as<int>(), c->ctr(), c->trial_ctr(), e0, e1, c->hread(), c->stream,
+                                          &herr);
+                HIPCHK(c, herr);
+            }
             c->host_sample_entries += (unsigned long long)nent;
             c->ev_kind[eslot] = nruns > 0 ? 1 : 0;
         }

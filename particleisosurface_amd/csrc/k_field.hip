@@ -1,6 +1,7 @@
 // Field evaluation at arbitrary points (Evaluator::SingleEval / SingleEvalWithGrad,
 // src/evaluator.cpp:60-125) and particle normals (CalcParticlesNormal, :363-375).
 #include "pisurf_internal.h"
+#include "point_eval.h"
 #include "run_eval.h"
 #include "run_tuner.h"
 #include "wave_eval.h"
@@ -9,120 +10,32 @@
 
 namespace pisurf {
 
-// SingleEval / SingleEvalWithGrad at points in any order: a wave takes m points (points_per_wave at most) one after another.
-// Lanes 0 - 8 look up the nine rows of a point's window, the lanes test 64 candidates at a time (consecutive
-// records of a row: coalesced reads, where threads with a point each gather from windows of their own), the
-// passing ones are listed in order in LDS and evaluated 64 at a time, and their terms wait in LDS until one lane
-// per sum adds them in the reference's order, the sums of all the wave's points side by side. Terms, order and
-// roundings are those of field_sum.
-//
-// What bounds it: the latency of a point's dependent reads, 16 waves per CU side by side (a thread per point's
-// window reads gathered a line per candidate: 1 M shuffled points with gradients on 1.6 M particles, compensated
-// FP32, 2216 -> 1157 us), and for a few points the latency of one: 1000 points 88 -> 8.4 us, as each point's
-// candidates are tested side by side instead of one by one.
-// (gradients in FP64 keep four points' terms: with eight, LDS leaves two workgroups per CU)
-constexpr int points_per_wave(bool fp64, bool grad) { return fp64 && grad ? 4 : 8; }
-
+// SingleEval / SingleEvalWithGrad, a wave per m points
+template <class R> struct PointSrc {
+    const float* q;
+    double* f;
+    double* grad;
+    R iso, sigma;
+    __device__ __forceinline__ bool point(int64_t i, float p[3]) const {
+        for (int a = 0; a < 3; a++) p[a] = q[3 * i + a];
+        return true;
+    }
+    __device__ __forceinline__ void store(int64_t i, int c, R v) const {
+        if (c == 0) f[i] = double(field_value(iso, sigma, v));
+        else grad[3 * i + c - 1] = double(sigma * v);
+    }
+};
 template <class R, bool K, bool GRAD, int MODE>
 __global__ void __launch_bounds__(256) k_eval_points(GridDev g, Recs<R> rec, FieldConst fc, const float* __restrict__ q,
                                                      int64_t n, int m, double* __restrict__ f,
                                                      double* __restrict__ grad, Counters* ctr) {
-    constexpr int C = GRAD ? 4 : 1, kStride = kWave + 1;  // (a stride of 64 would put every sum's terms in one bank)
-    __shared__ R terms[4][points_per_wave(sizeof(R) == 8, GRAD) * C * kStride];
-    __shared__ int listed[4][2 * kWave];
+    __shared__ PointLds<R, GRAD> lds[4];
     const int lane = threadIdx.x & (kWave - 1), w = threadIdx.x / kWave;
-    R* const term = terms[w];
-    int* const list = listed[w];
     const int64_t i0 = ((int64_t)blockIdx.x * 4 + w) * m;
-    const int np = (int)max((int64_t)0, min((int64_t)m, n - i0));  // uniform over the wave
-    const R inv_h2 = R(fc.inv_h2), h2 = R(fc.h2);
-    Acc<R, K> sum;    // lane k C + c: sum c of point k
-    int waiting = 0;  // its terms not added yet
-    auto add_terms = [&]() {
-        int most = waiting;
-#pragma unroll
-        for (int o = 32; o > 0; o >>= 1) most = max(most, __shfl_xor(most, o, kWave));
-        for (int t = 0; t < most; t++)
-            if (t < waiting) sum.add_unfused(term[lane * kStride + t]);
-        waiting = 0;
-        wave_sync();
-    };
-    unsigned long long vis = 0;
-    for (int k = 0; k < np; k++) {
-        const float x = q[3 * (i0 + k)], y = q[3 * (i0 + k) + 1], z = q[3 * (i0 + k) + 2];
-        const R px = R(x), py = R(y), pz = R(z);
-        int ix, iy, iz, lo = 0, hi = 0;
-        cell_of(g, x, y, z, ix, iy, iz);
-        if (lane >= 9 || !row_range(g, ix, iy, iz, lane, lo, hi)) lo = hi = 0;
-        int end = hi - lo;
-#pragma unroll
-        for (int o = 1; o < 16; o <<= 1) {
-            const int t = __shfl_up(end, o, kWave);
-            end += lane >= o ? t : 0;
-        }
-        // row r holds positions [first[r], first[r + 1]) of the window, position t being sorted particle t + d[r]
-        const int begin = end - (hi - lo);
-        int first[9], d[9];
-#pragma unroll
-        for (int r = 0; r < 9; r++) {
-            first[r] = __builtin_amdgcn_readlane(begin, r);
-            d[r] = __builtin_amdgcn_readlane(lo - begin, r);
-        }
-        const int total = __builtin_amdgcn_readlane(end, 8);
-        vis += (unsigned long long)total;
-        int have = 0;  // listed candidates
-        auto evaluate = [&](int cnt) {
-            if (__any(waiting && lane / C == k)) add_terms();  // the point's earlier terms come first
-            if (lane < cnt) {
-                const int j = list[lane];
-                const auto a = rec.a[j];
-                const float4 l4 = (K && sizeof(R) == 4) ? fc.lo[j] : make_float4(0.f, 0.f, 0.f, 0.f);
-                const R dx = px - a.x, dy = py - a.y, dz = pz - a.z;
-                Acc<R, K> v, gv[3];
-                field_contrib<R, K, GRAD, MODE>(fc, inv_h2, h2, dx, dy, dz, dist2(dx, dy, dz), rec.g[2 * j],
-                                                rec.g[2 * j + 1], l4, v, gv);
-                term[(k * C) * kStride + lane] = v.get();
-                if (GRAD)
-#pragma unroll
-                    for (int c = 0; c < 3; c++) term[(k * C + (GRAD ? 1 + c : 0)) * kStride + lane] = gv[c].get();
-            }
-            wave_sync();
-            if (lane / C == k) waiting = cnt;
-        };
-        for (int t0 = 0; t0 < total; t0 += kWave) {
-            const int t = t0 + lane;
-            int dt = d[0];
-#pragma unroll
-            for (int r = 1; r < 9; r++) dt = t >= first[r] ? d[r] : dt;
-            bool pass = false;
-            if (t < total) {
-                const auto a = rec.a[t + dt];
-                pass = !(dist2(px - a.x, py - a.y, pz - a.z) >= a.w);
-            }
-            const unsigned long long pm = __ballot(pass);
-            if (pass) list[have + __builtin_popcountll(pm & ((1ull << lane) - 1ull))] = t + dt;
-            have += __builtin_popcountll(pm);
-            wave_sync();
-            if (have >= kWave) {
-                evaluate(kWave);
-                // the rest moves to the front
-                const int rest = lane + kWave < have ? list[kWave + lane] : 0;
-                wave_sync();
-                if (lane + kWave < have) list[lane] = rest;
-                have -= kWave;
-                wave_sync();
-            }
-        }
-        if (have) evaluate(have);
-    }
-    add_terms();
-    if (lane < np * C) {
-        const int64_t i = i0 + lane / C;
-        const R sigma = out_sigma<R, K>(fc);
-        const int c = lane % C;
-        if (c == 0) f[i] = double(field_value(R(fc.iso), sigma, sum.get()));
-        else grad[3 * i + c - 1] = double(sigma * sum.get());
-    }
+    const int np = (int)max((int64_t)0, min((int64_t)m, n - i0));
+    const PointSrc<R> src{q, f, grad, R(fc.iso), out_sigma<R, K>(fc)};
+    int evals = 0;
+    const unsigned long long vis = point_eval<R, K, GRAD, MODE>(g, rec, fc, src, i0, np, lds[w], evals);
     Counters* ct = ctr_stripe(ctr);
     if (lane == 0 && np > 0) {
         atomicAdd(GRAD ? &ct->grad_evals : &ct->field_evals, (unsigned long long)np);
@@ -182,9 +95,7 @@ __global__ void __launch_bounds__(T) k_run_normals(GridDev g, Recs<R> rec, Field
 void launch_eval_points(int prec, GridDev g, const void* ra, const void* rg, FieldConst fc, const float* q, int64_t n,
                         double* f, double* grad, Counters* ctr, hipStream_t s) {
     if (n <= 0) return;
-    // points per wave: one as long as the waves fit the chip at once (256 CUs x 16), for the latency of few
-    // points, then as many as share their sums' additions
-    const int m = (int)std::min<int64_t>(points_per_wave(prec == 2, grad != nullptr), (n + 4095) / 4096);
+    const int m = point_share(n, points_per_wave(prec == 2, grad != nullptr));
     const unsigned nb = (unsigned)((n + 4 * m - 1) / (4 * m));
     auto go = [&](auto gr, auto mode) {
         constexpr bool G = decltype(gr)::value;
@@ -198,12 +109,10 @@ void launch_eval_points(int prec, GridDev g, const void* ra, const void* rg, Fie
             else k_eval_points<float, false, G, M><<<nb, 256, 0, s>>>(g, r, fc, q, n, m, f, grad, ctr);
         }
     };
-    auto with = [&](auto gr) {
-        if (field_mode(fc) == kModeAniBspline) go(gr, std::integral_constant<int, kModeAniBspline>());
-        else go(gr, std::integral_constant<int, kModeAny>());
-    };
-    if (grad) with(std::true_type());
-    else with(std::false_type());
+    point_dispatch(field_mode(fc), [&](auto mode) {
+        if (grad) go(std::true_type(), mode);
+        else go(std::false_type(), mode);
+    });
 }
 
 // Many points: sorted by hash cell, then 64 to a wave (wave_eval.h)
@@ -225,11 +134,12 @@ template <class R> struct QuerySrc {
     double* f;
     double* grad;
     R iso, sigma;
-    __device__ __forceinline__ void point(int h, float p[3]) const {
+    __device__ __forceinline__ bool point(int h, float p[3]) const {
         const float* x = q + 3 * (int64_t)kv.val(h);
         p[0] = x[0];
         p[1] = x[1];
         p[2] = x[2];
+        return true;
     }
     __device__ __forceinline__ void store(int h, R sum, const R* gr) const {
         const int64_t i = kv.val(h);

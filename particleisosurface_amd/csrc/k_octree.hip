@@ -4,6 +4,7 @@
 #include <climits>
 
 #include "pisurf_internal.h"
+#include "point_eval.h"
 #include "qef_device.h"
 #include "run_eval.h"
 #include "run_tuner.h"
@@ -372,11 +373,12 @@ template <class R> struct CenterSrc {
     SortedKV kv;
     R* samples;
     R iso, sigma;
-    __device__ __forceinline__ void point(int h, float p[3]) const {
+    __device__ __forceinline__ bool point(int h, float p[3]) const {
         const float4 c = lv.c[list[kv.val(h)]];
         p[0] = c.x;
         p[1] = c.y;
         p[2] = c.z;
+        return true;
     }
     __device__ __forceinline__ void store(int h, R sum, const R*) const {
         samples[(int64_t)list[kv.val(h)] * 27 + 13] = field_value(iso, sigma, sum);
@@ -459,42 +461,66 @@ static int build_run_starts(GridDev g, SortedKV kv, int gshift, const int* hlist
     return nr;
 }
 
-// ---- sample points merged per tile of nodes, before the global sort -------------------------
+// ---- sample points merged per tile of nodes -------------------------------------------------
 // The listed nodes of a level (one node size) are taken in tiles of 256 consecutive list entries
 // (children follow their parents, so a tile is mostly a compact piece of space). Sample s of node
 // ip lies on lattice point 2 ip + t(s), t(s) in {0, 1, 2}^3; the nodes that can share it are
 // ip + d with d_a in {-1, 0} when t_a = 0, {0} when t_a = 1 and {0, +1} when t_a = 2. Of those,
-// the ones with a -1 component (the others come later in Morton order) are looked up in a dense
-// LDS map over the tile's bounding box, and the entry refers to the one first in the list, if it
-// is earlier than the entry's own node and that sample's coordinates are bitwise identical to its
-// own. References point to earlier nodes, so following them ends at an entry with none, which owns
-// a record; the global heads pass, which compares coordinates, still merges identical points of
-// different records. A tile whose box (grown by one) exceeds the map gives every entry its own
-// record. A tile takes the slots of its records from a level-wide counter (*nrec, one atomic per
-// tile) and writes per record its sort key as k_sample_keys makes it (packed with the slot when
-// vbits > 0, else the slot in rval) and node * 27 + sample of the owning entry (rent), per entry
-// the slot of its record (ent_rec). The order of the tiles' slot ranges varies from run to run;
-// what is evaluated does not: equal points get equal values whichever record is their head.
+// the ones with a -1 component (the others come later in Morton order) are looked up in a hash
+// table of the tile's nodes, and the entry refers to the one first in the list, if it is earlier than the
+// entry's own node and that sample's coordinates are bitwise identical to its own. References point to
+// earlier nodes, so following them ends at an entry with none, which owns a record. A tile takes the slots
+// of its records from a level-wide counter (*nrec, one atomic per tile) and writes per record node * 27 +
+// sample of the owning entry (rent), per entry the slot of its record (ent_rec). The order of the tiles'
+// slot ranges varies from run to run; what is evaluated does not: equal points get equal values.
+//
+// LOCAL: the records are evaluated as they are. A tile's slots are grouped by hash cell, x fastest (a count
+// per cell of the tile's box, taken modulo kStBuckets, then a place per record), and padded to whole waves with
+// rent = -1. A point on the border of two tiles is evaluated by both: 1.15 - 1.3 times the level's distinct points.
+// Otherwise the records are sorted and merged over the whole level: the tile writes each record's sort key
+// as k_sample_keys makes it (packed with the slot when vbits > 0, else the slot in rval).
+//
+// What a level-wide sort saved in evaluations (a sixth) it spent on four to six radix passes over the records, the
+// search for equal neighbours and the lists of heads, cells and runs: the tree of a 1.1 M-particle crown splash with QEF
+// vertices (44.9 M distinct points at its deepest level, compensated FP32) takes 12.1 ms instead of 15.6, of
+// 4 M particles 5.3 instead of 5.9, of 12 M 9.9 instead of 12.4, and a 14 k-particle frame, which waits for launches,
+// 0.61 instead of 0.95 (164 launches a frame instead of 232). A box map of 4096 node cells in place of
+// the hash table left tiles that straddle octants unmerged: 1.29 - 1.42 times the distinct points at the
+// deepest levels.
 constexpr int kStT = 256;           // nodes per tile
 constexpr int kStRecs = 27 * kStT;  // records per tile at most
-constexpr int kStMap = 4096;        // dense map cells
+constexpr int kStTable = 1024;      // slots of the hash table of nodes
+constexpr int kStBuckets = 2048;    // cells told apart in a tile
 
+__device__ __forceinline__ uint64_t node_key(int x, int y, int z) {
+    return (uint64_t)(uint32_t)(x & 0x1fffff) | ((uint64_t)(uint32_t)(y & 0x1fffff) << 21) |
+           ((uint64_t)(uint32_t)(z & 0x1fffff) << 42);
+}
+__device__ __forceinline__ unsigned node_hash(uint64_t k) {
+    return (unsigned)((k * 0x9e3779b97f4a7c15ull) >> 54) & (kStTable - 1);
+}
+
+template <bool LOCAL>
 __global__ void __launch_bounds__(kStT) k_sample_tiles(GridDev g, NodeLevel lv, const int* __restrict__ list,
                                                        int64_t k, float ox, float oy, float oz, int lb, int vbits,
                                                        int* __restrict__ nrec, int* __restrict__ ent_rec,
                                                        uint64_t* __restrict__ rkey, int* __restrict__ rval,
                                                        int* __restrict__ rent) {
-    __shared__ short map[kStMap];
+    __shared__ int table[kStTable];   // node of the tile, or -1
+    __shared__ uint64_t nkey[kStT];
     __shared__ float4 cen[kStT];
     __shared__ int nid[kStT];
-    __shared__ short ref[kStRecs];    // per tile entry (node * 27 + sample): the entry it refers to, or -1
-    __shared__ short recid[kStRecs];  // record of an entry that owns one
+    __shared__ short ref[kStRecs];  // per tile entry (node * 27 + sample): the entry it refers to, or ~its record
+    __shared__ int bucket[LOCAL ? kStBuckets : 1];
     __shared__ int red[6][kStT / kWave];
     __shared__ int wsum[kStT / kWave];
     __shared__ int tbase;
     const int t = threadIdx.x, lane = t & (kWave - 1), w = t / kWave;
     const int64_t l0 = (int64_t)blockIdx.x * kStT, li = l0 + t;
     const bool act = li < k;
+    for (int q = t; q < kStTable; q += kStT) table[q] = -1;
+    if (LOCAL)
+        for (int q = t; q < kStBuckets; q += kStT) bucket[q] = 0;
     int4 ip = make_int4(0, 0, 0, 0);
     float4 c = make_float4(0.f, 0.f, 0.f, 0.f);
     if (act) {
@@ -503,65 +529,98 @@ __global__ void __launch_bounds__(kStT) k_sample_tiles(GridDev g, NodeLevel lv, 
         ip = lv.ip[node];
         cen[t] = c;
         nid[t] = node;
+        nkey[t] = node_key(ip.x, ip.y, ip.z);
     }
-    // the tile's bounding box of node coordinates
-    int mn[3] = {act ? ip.x : INT_MAX, act ? ip.y : INT_MAX, act ? ip.z : INT_MAX};
-    int mx[3] = {act ? ip.x : INT_MIN, act ? ip.y : INT_MIN, act ? ip.z : INT_MIN};
-#pragma unroll
-    for (int a = 0; a < 3; a++)
-#pragma unroll
-        for (int o = 32; o > 0; o >>= 1) {
-            mn[a] = min(mn[a], __shfl_xor(mn[a], o, kWave));
-            mx[a] = max(mx[a], __shfl_xor(mx[a], o, kWave));
+    int box[6] = {0, 0, 0, 0, 0, 0};  // LOCAL: first cell and dimensions of the tile's box
+    if (LOCAL) {
+        // its corners are corner samples of nodes
+        int mn[3] = {INT_MAX, INT_MAX, INT_MAX}, mx[3] = {INT_MIN, INT_MIN, INT_MIN};
+        if (act) {
+            float p[3];
+            sample_point(c, 0, p);
+            cell_of(g, p[0], p[1], p[2], mn[0], mn[1], mn[2]);
+            sample_point(c, 26, p);
+            cell_of(g, p[0], p[1], p[2], mx[0], mx[1], mx[2]);
         }
-    if (lane == 0)
+#pragma unroll
+        for (int a = 0; a < 3; a++)
+#pragma unroll
+            for (int o = 32; o > 0; o >>= 1) {
+                mn[a] = min(mn[a], __shfl_xor(mn[a], o, kWave));
+                mx[a] = max(mx[a], __shfl_xor(mx[a], o, kWave));
+            }
+        if (lane == 0)
+            for (int a = 0; a < 3; a++) {
+                red[a][w] = mn[a];
+                red[3 + a][w] = mx[a];
+            }
+    }
+    __syncthreads();
+    if (LOCAL) {
+#pragma unroll
         for (int a = 0; a < 3; a++) {
-            red[a][w] = mn[a];
-            red[3 + a][w] = mx[a];
+            int lo = red[a][0], hi = red[3 + a][0];
+            for (int q = 1; q < kStT / kWave; q++) {
+                lo = min(lo, red[a][q]);
+                hi = max(hi, red[3 + a][q]);
+            }
+            box[a] = lo;
+            box[3 + a] = (int)((unsigned)hi - (unsigned)lo + 1u);
         }
-    for (int q = t; q < kStMap; q += kStT) map[q] = -1;
-    __syncthreads();
-    int b0[3], dim[3];
-    bool dense = true;  // uniform over the tile
-#pragma unroll
-    for (int a = 0; a < 3; a++) {
-        int lo = red[a][0], hi = red[3 + a][0];
-        for (int q = 1; q < kStT / kWave; q++) {
-            lo = min(lo, red[a][q]);
-            hi = max(hi, red[3 + a][q]);
-        }
-        b0[a] = lo - 1;  // one node of margin: the neighbours looked up
-        dim[a] = hi - lo + 3;
-        if (dim[a] > kStMap) dense = false;
     }
-    if (dense && dim[0] * dim[1] * dim[2] > kStMap) dense = false;
-    if (dense && act) map[(ip.x - b0[0]) + dim[0] * ((ip.y - b0[1]) + dim[1] * (ip.z - b0[2]))] = (short)t;
+    if (act)
+        for (unsigned h = node_hash(nkey[t]);; h = (h + 1) & (kStTable - 1))
+            if (atomicCAS(&table[h], -1, t) == -1) break;  // at most kStT of kStTable slots are taken
     __syncthreads();
-    int own = 0;
+    auto bucket_of = [&](int sm) {
+        float p[3];
+        int ix, iy, iz;
+        sample_point(c, sm, p);
+        cell_of(g, p[0], p[1], p[2], ix, iy, iz);
+        const unsigned i = ((unsigned)iz - (unsigned)box[2]) * (unsigned)box[4] + ((unsigned)iy - (unsigned)box[1]);
+        return (int)((i * (unsigned)box[3] + ((unsigned)ix - (unsigned)box[0])) % kStBuckets);
+    };
+    unsigned owner = 0;  // samples of this node that own a record
     if (act) {
-        const int m0 = (ip.x - b0[0]) + dim[0] * ((ip.y - b0[1]) + dim[1] * (ip.z - b0[2]));
+        // the neighbours with a -1 component: (d_x + 1) + 3 (d_y + 1) + 9 (d_z + 1)
+        short nb[27];
+#pragma unroll
+        for (int d = 0; d < 27; d++) {
+            const int dx = d % 3 - 1, dy = (d / 3) % 3 - 1, dz = d / 9 - 1;
+            int found = -1;
+            if (dx < 0 || dy < 0 || dz < 0) {
+                const uint64_t key = node_key(ip.x + dx, ip.y + dy, ip.z + dz);
+                for (unsigned h = node_hash(key);; h = (h + 1) & (kStTable - 1)) {
+                    const int j = table[h];
+                    if (j < 0) break;
+                    if (nkey[j] == key) {
+                        found = j;
+                        break;
+                    }
+                }
+            }
+            nb[d] = (short)found;
+        }
 #pragma unroll
         for (int sm = 0; sm < 27; sm++) {
             const int ta[3] = {sm % 3, (sm / 3) % 3, sm / 9};
             int best = t, bs = sm;
-            if (dense) {
 #pragma unroll
-                for (int d = 1; d < 8; d++) {
-                    int dd[3];
-                    bool ok = true, earlier = false;
+            for (int d = 1; d < 8; d++) {
+                int dd[3];
+                bool ok = true, earlier = false;
 #pragma unroll
-                    for (int a = 0; a < 3; a++) {
-                        const int bit = (d >> a) & 1;
-                        dd[a] = bit ? (ta[a] == 0 ? -1 : (ta[a] == 2 ? 1 : 0)) : 0;
-                        if (bit && dd[a] == 0) ok = false;
-                        if (dd[a] < 0) earlier = true;
-                    }
-                    if (!ok || !earlier) continue;
-                    const int j = map[m0 + dd[0] + dim[0] * (dd[1] + dim[1] * dd[2])];
-                    if (j >= 0 && j < best) {
-                        best = j;
-                        bs = (ta[0] - 2 * dd[0]) + 3 * (ta[1] - 2 * dd[1]) + 9 * (ta[2] - 2 * dd[2]);
-                    }
+                for (int a = 0; a < 3; a++) {
+                    const int bit = (d >> a) & 1;
+                    dd[a] = bit ? (ta[a] == 0 ? -1 : (ta[a] == 2 ? 1 : 0)) : 0;
+                    if (bit && dd[a] == 0) ok = false;
+                    if (dd[a] < 0) earlier = true;
+                }
+                if (!ok || !earlier) continue;
+                const int j = nb[(dd[0] + 1) + 3 * (dd[1] + 1) + 9 * (dd[2] + 1)];
+                if (j >= 0 && j < best) {
+                    best = j;
+                    bs = (ta[0] - 2 * dd[0]) + 3 * (ta[1] - 2 * dd[1]) + 9 * (ta[2] - 2 * dd[2]);
                 }
             }
             short r = -1;
@@ -572,10 +631,19 @@ __global__ void __launch_bounds__(kStT) k_sample_tiles(GridDev g, NodeLevel lv, 
                 if (same_point(p, q)) r = (short)(best * 27 + bs);
             }
             ref[t * 27 + sm] = r;
-            own += r < 0 ? 1 : 0;
+            owner |= r < 0 ? 1u << sm : 0u;
+            if (LOCAL && r < 0) atomicAdd(&bucket[bucket_of(sm)], 1);
         }
     }
-    // records numbered in entry order (thread, then sample)
+    // records numbered in entry order (thread, then sample), or LOCAL bucket by bucket
+    constexpr int kPer = kStBuckets / kStT;
+    int own = __builtin_popcount(owner);
+    if (LOCAL) {
+        __syncthreads();
+        own = 0;
+#pragma unroll
+        for (int i = 0; i < kPer; i++) own += bucket[t * kPer + i];
+    }
     const int incl = wave_incl_scan(own, lane);
     if (lane == kWave - 1) wsum[w] = incl;
     __syncthreads();
@@ -585,21 +653,39 @@ __global__ void __launch_bounds__(kStT) k_sample_tiles(GridDev g, NodeLevel lv, 
         if (q < w) u += wsum[q];
         total += wsum[q];
     }
-    if (t == 0) tbase = atomicAdd(nrec, total);
-    if (act)
-        for (int sm = 0; sm < 27; sm++)
-            if (ref[t * 27 + sm] < 0) recid[t * 27 + sm] = (short)u++;
+    const int padded = LOCAL ? (total + kWave - 1) & ~(kWave - 1) : total;
+    if (t == 0) tbase = atomicAdd(nrec, padded);
+    if (LOCAL) {
+#pragma unroll
+        for (int i = 0; i < kPer; i++) {
+            const int n = bucket[t * kPer + i];
+            bucket[t * kPer + i] = u;
+            u += n;
+        }
+    }
+    __syncthreads();
+    if (LOCAL) {
+        for (unsigned m = owner; m; m &= m - 1) {
+            const int sm = __builtin_ctz(m), slot = atomicAdd(&bucket[bucket_of(sm)], 1);
+            ref[t * 27 + sm] = (short)~slot;
+            rent[tbase + slot] = nid[t] * 27 + sm;
+        }
+        if (total + t < padded) rent[tbase + total + t] = -1;
+    } else {
+        for (unsigned m = owner; m; m &= m - 1) ref[t * 27 + __builtin_ctz(m)] = (short)~(u++);
+    }
     __syncthreads();
     // entry by entry (coalesced): the record slot of every entry, the key and entry of every record
     const int ne = (int)min<int64_t>(k - l0, kStT) * 27;
     const float o[3] = {ox, oy, oz};
     const uint32_t m = (1u << lb) - 1;
     for (int e = t; e < ne; e += kStT) {
-        int r = e;
-        while (ref[r] >= 0) r = ref[r];
-        const int slot = tbase + recid[r];
+        int r = ref[e];
+        const bool owns = r < 0;
+        while (r >= 0) r = ref[r];
+        const int slot = tbase + ~r;
         ent_rec[l0 * 27 + e] = slot;
-        if (r != e) continue;
+        if (LOCAL || !owns) continue;
         const float4 cc = cen[e / 27];
         float p[3];
         sample_point(cc, e % 27, p);
@@ -632,14 +718,14 @@ __global__ void k_record_heads(SortedKV kv, const int* __restrict__ rep, const i
     rec_head[kv.val(j)] = hpos[r];
 }
 
-// every sample entry receives its point's value
+// every sample entry receives its point's value (rec_head NULL: the records are the points)
 __global__ void k_entry_scatter(const int* __restrict__ list, const int* __restrict__ ent_rec,
                                 const int* __restrict__ rec_head, int64_t nent, const void* __restrict__ vals, int rsz,
                                 void* __restrict__ samples) {
     const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (e >= nent) return;
     const int64_t dst = (int64_t)list[e / 27] * 27 + e % 27;
-    const int64_t src = rec_head[ent_rec[e]];
+    const int64_t src = rec_head ? rec_head[ent_rec[e]] : ent_rec[e];
     if (rsz == 8) ((double*)samples)[dst] = ((const double*)vals)[src];
     else ((float*)samples)[dst] = ((const float*)vals)[src];
 }
@@ -648,9 +734,70 @@ void launch_sample_tiles(GridDev g, NodeLevel lv, const int* list, int64_t k, co
                          int vbits, int* nrec, int* ent_rec, uint64_t* rkey, int* rval, int* rent, hipStream_t s) {
     launch_fill_i32(nrec, 1, 0, s);
     if (k > 0)
-        k_sample_tiles<<<(unsigned)((k + kStT - 1) / kStT), kStT, 0, s>>>(g, lv, list, k, origin[0], origin[1],
-                                                                        origin[2], lb, vbits, nrec, ent_rec, rkey,
-                                                                        rval, rent);
+        k_sample_tiles<false><<<(unsigned)((k + kStT - 1) / kStT), kStT, 0, s>>>(
+            g, lv, list, k, origin[0], origin[1], origin[2], lb, vbits, nrec, ent_rec, rkey, rval, rent);
+}
+
+// records of the tiles (k_sample_tiles<true>): slot h is sample rent[h] % 27 of node rent[h] / 27, or unused
+template <class R> struct TileSrc {
+    NodeLevel lv;
+    const int* rent;
+    R* out;
+    R iso, sigma;
+    __device__ __forceinline__ bool point(int64_t h, float p[3]) const {
+        const int ns = rent[h];
+        if (ns < 0) return false;
+        sample_point(lv.c[ns / 27], ns % 27, p);
+        return true;
+    }
+    __device__ __forceinline__ void store(int64_t h, R sum, const R*) const { out[h] = field_value(iso, sigma, sum); }
+    __device__ __forceinline__ void store(int64_t h, int, R sum) const { out[h] = field_value(iso, sigma, sum); }
+};
+
+__device__ __forceinline__ void count_samples(Counters* c, unsigned long long n) {
+    atomicAdd(&c->sample_unique, n);
+    atomicAdd(&c->run_evals, n);
+}
+
+// The records evaluated 64 to a wave. The grid covers the level's entries; records end at *nrec.
+template <class R, bool K, int T, int MODE>
+__global__ void __launch_bounds__(T) k_wave_samples(GridDev g, Recs<R> rec, FieldConst fc, NodeLevel lv,
+                                                    const int* __restrict__ rent, const int* __restrict__ nrec,
+                                                    R* __restrict__ out, Counters* ctr) {
+    __shared__ WaveLds<WaveField<R, K, false, MODE>> lds[T / kWave];
+    const int n = *nrec;
+    if ((int)blockIdx.x * T >= n) return;  // uniform over the block
+    const TileSrc<R> src{lv, rent, out, R(fc.iso), out_sigma<R, K>(fc)};
+    const unsigned long long vis = wave_eval<T, R, K, false, MODE, 0>(g, rec, fc, src, n, lds);
+    Counters* c = ctr_stripe(ctr);
+    wave_count(&c->sample_candidates, vis);
+    wave_count(&c->candidates, vis);
+    wave_count(&c->run_candidates, vis);
+    const int h = (int)blockIdx.x * T + (int)threadIdx.x;
+    const int m = __builtin_popcountll(__ballot(h < n && rent[min(h, n - 1)] >= 0));
+    if ((threadIdx.x & (kWave - 1)) == 0 && m) count_samples(c, (unsigned long long)m);
+}
+
+// The records evaluated by a wave per m points
+template <class R, bool K, int MODE>
+__global__ void __launch_bounds__(256) k_point_samples(GridDev g, Recs<R> rec, FieldConst fc, NodeLevel lv,
+                                                       const int* __restrict__ rent, const int* __restrict__ nrec,
+                                                       int m, R* __restrict__ out, Counters* ctr) {
+    __shared__ PointLds<R, false> lds[4];
+    const int64_t n = *nrec;
+    const int w = threadIdx.x / kWave;
+    const int64_t i0 = ((int64_t)blockIdx.x * 4 + w) * m;
+    const int np = (int)max((int64_t)0, min((int64_t)m, n - i0));
+    const TileSrc<R> src{lv, rent, out, R(fc.iso), out_sigma<R, K>(fc)};
+    int evals = 0;
+    const unsigned long long vis = point_eval<R, K, false, MODE>(g, rec, fc, src, i0, np, lds[w], evals);
+    if ((threadIdx.x & (kWave - 1)) == 0 && evals > 0) {
+        Counters* c = ctr_stripe(ctr);
+        atomicAdd(&c->sample_candidates, vis);
+        atomicAdd(&c->candidates, vis);
+        atomicAdd(&c->run_candidates, vis);
+        count_samples(c, (unsigned long long)evals);
+    }
 }
 
 // distinct sample points of a level (cell-major), evaluated run by run
@@ -683,26 +830,6 @@ __global__ void __launch_bounds__(T) k_run_samples(GridDev g, Recs<R> rec, Field
     if (threadIdx.x == 0) {
         atomicAdd(&c->sample_unique, (unsigned long long)(h1 - h0));
         atomicAdd(&c->run_evals, (unsigned long long)(h1 - h0));
-    }
-}
-
-// the same with 64 consecutive points (in cell order) per wave
-template <class R, bool K, int T, int MODE>
-__global__ void __launch_bounds__(T) k_wave_samples(GridDev g, Recs<R> rec, FieldConst fc, NodeLevel lv,
-                                                    const int* __restrict__ list, SortedKV kv,
-                                                    const int* __restrict__ hlist, int n, R* __restrict__ out,
-                                                    const int* __restrict__ ent, Counters* ctr) {
-    __shared__ WaveLds<WaveField<R, K, false, MODE>> lds[T / kWave];
-    const SampleSrc<R> src{lv, list, kv, hlist, out, R(fc.iso), out_sigma<R, K>(fc), ent};
-    const unsigned long long vis = wave_eval<T, R, K, false, MODE>(g, rec, fc, src, n, lds);
-    Counters* c = ctr_stripe(ctr);
-    wave_count(&c->sample_candidates, vis);
-    wave_count(&c->candidates, vis);
-    wave_count(&c->run_candidates, vis);
-    if (threadIdx.x == 0) {
-        const unsigned long long m = (unsigned long long)min(T, n - (int)blockIdx.x * T);
-        atomicAdd(&c->sample_unique, m);
-        atomicAdd(&c->run_evals, m);
     }
 }
 
@@ -1122,30 +1249,75 @@ static void launch_run_samples(int prec, int T, GridDev g, const void* ra, const
 }
 
 // one launch of the sample waves
-static void launch_wave_samples(int prec, int T, GridDev g, const void* ra, const void* rg, FieldConst fc, NodeLevel lv,
-                                const int* list, SortedKV kv, const int* hlist, int nh, void* vals, const int* ent,
-                                Counters* ctr, hipStream_t s) {
-    const unsigned nb = (unsigned)((nh + T - 1) / T);
-    wave_dispatch(T, field_mode(fc), [&](auto tag, auto mode) {
-        constexpr int TT = decltype(tag)::value, M = decltype(mode)::value;
-        if (prec == 2) {
-            Recs<double> r{(const double4*)ra, (const double4*)rg};
-            k_wave_samples<double, false, TT, M><<<nb, TT, 0, s>>>(g, r, fc, lv, list, kv, hlist, nh, (double*)vals, ent,
-                                                                   ctr);
-        } else {
-            Recs<float> r{(const float4*)ra, (const float4*)rg};
-            if (prec == 1)
-                k_wave_samples<float, true, TT, M><<<nb, TT, 0, s>>>(g, r, fc, lv, list, kv, hlist, nh, (float*)vals,
-                                                                     ent, ctr);
-            else
-                k_wave_samples<float, false, TT, M><<<nb, TT, 0, s>>>(g, r, fc, lv, list, kv, hlist, nh, (float*)vals,
-                                                                      ent, ctr);
-        }
-    });
+// Levels of 8 and more points per hash cell are merged per tile and, from kWaveNodes nodes on (about 70 k points),
+// evaluated 64 to a wave; fewer, by a wave per few points, as such a launch lasts as long as its slowest wave (three
+// levels of a 14 k-particle frame, 7834 nodes the last: 0.12 ms with that one as waves, 0.15 ms without). At 1
+// point per cell (D_min) a wave's points share no window: levels of fewer than kTileNodes nodes go point by point,
+// larger ones are sorted over the level and evaluated by runs. Point by point at all sizes, a frame took 0.23 ms
+// longer with 79 k nodes there, 0.97 ms with 245 k, and the same with 33 k.
+constexpr int64_t kWaveNodes = 1 << 12;
+constexpr int64_t kTileNodes = 1 << 15;
+bool samples_by_tile(int64_t k, double density) {
+    return tile_record_bound(k) < INT32_MAX && (density >= kWaveDensity || k < kTileNodes);
+}
+
+void launch_samples_by_tile(int prec, GridDev g, const void* ra, const void* rg, FieldConst fc, NodeLevel lv,
+                            const int* list, int64_t k, double density, int* nrec, int* ent_rec, int* rent, void* vals,
+                            void* samples, Counters* ctr, Counters* trial_ctr, hipEvent_t e0, hipEvent_t e1,
+                            hipStream_t s) {
+    const unsigned tiles = (unsigned)((k + kStT - 1) / kStT);
+    launch_fill_i32(nrec, 1, 0, s);
+    k_sample_tiles<true><<<tiles, kStT, 0, s>>>(g, lv, list, k, 0.f, 0.f, 0.f, 0, 0, nrec, ent_rec, nullptr, nullptr,
+                                                rent);
+    const int64_t most = tile_record_bound(k);
+    (void)hipEventRecord(e0, s);
+    if (density >= kWaveDensity && k >= kWaveNodes) {
+        tuned_run_launch(
+            prec, kRunSamples, density, true, trial_ctr, s, [](RunShape) { return true; },
+            [&](RunShape c, bool trial) {
+                Counters* cc = trial ? trial_ctr : ctr;
+                const unsigned nb = (unsigned)((most + c.T - 1) / c.T);
+                wave_dispatch(c.T, field_mode(fc), [&](auto tag, auto mode) {
+                    constexpr int TT = decltype(tag)::value, M = decltype(mode)::value;
+                    if (prec == 2) {
+                        Recs<double> r{(const double4*)ra, (const double4*)rg};
+                        k_wave_samples<double, false, TT, M><<<nb, TT, 0, s>>>(g, r, fc, lv, rent, nrec,
+                                                                               (double*)vals, cc);
+                    } else {
+                        Recs<float> r{(const float4*)ra, (const float4*)rg};
+                        if (prec == 1)
+                            k_wave_samples<float, true, TT, M><<<nb, TT, 0, s>>>(g, r, fc, lv, rent, nrec,
+                                                                                 (float*)vals, cc);
+                        else
+                            k_wave_samples<float, false, TT, M><<<nb, TT, 0, s>>>(g, r, fc, lv, rent, nrec,
+                                                                                  (float*)vals, cc);
+                    }
+                });
+            });
+    } else {
+        const int m = point_share(most, points_per_wave(prec == 2, false));
+        const unsigned nb = (unsigned)((most + 4 * m - 1) / (4 * m));
+        point_dispatch(field_mode(fc), [&](auto mode) {
+            constexpr int M = decltype(mode)::value;
+            if (prec == 2) {
+                Recs<double> r{(const double4*)ra, (const double4*)rg};
+                k_point_samples<double, false, M><<<nb, 256, 0, s>>>(g, r, fc, lv, rent, nrec, m, (double*)vals, ctr);
+            } else {
+                Recs<float> r{(const float4*)ra, (const float4*)rg};
+                if (prec == 1)
+                    k_point_samples<float, true, M><<<nb, 256, 0, s>>>(g, r, fc, lv, rent, nrec, m, (float*)vals, ctr);
+                else
+                    k_point_samples<float, false, M><<<nb, 256, 0, s>>>(g, r, fc, lv, rent, nrec, m, (float*)vals, ctr);
+            }
+        });
+    }
+    (void)hipEventRecord(e1, s);
+    k_entry_scatter<<<(unsigned)((27 * k + 255) / 256), 256, 0, s>>>(list, ent_rec, nullptr, 27 * k, vals,
+                                                                     prec == 2 ? 8 : 4, samples);
 }
 
 void launch_sample_dedupe_eval(int prec, GridDev g, const void* ra, const void* rg, FieldConst fc, NodeLevel lv,
-                               const int* list, SortedKV kv, const int* ent, int gshift, double density, int64_t nrec,
+                               const int* list, SortedKV kv, const int* ent, int gshift, int64_t nrec,
                                const int* ent_rec, int64_t nent, int* rec_head, int* head, int* hpos, int* rep,
                                int* hlist, int* cwork, int64_t* nheads_out, int64_t* nruns_out, int* kx_out,
                                void* vals, void* samples, int* tmp, Counters* ctr, Counters* trial_ctr, hipEvent_t e0,
@@ -1170,31 +1342,20 @@ void launch_sample_dedupe_eval(int prec, GridDev g, const void* ra, const void* 
     *nheads_out = nh;
     int* rstart = nullptr;
     int nr = 0;
-    if (density >= kWaveDensity && nh >= kWaveMin) {
-        (void)hipEventRecord(e0, s);
-        tuned_run_launch(
-            prec, kRunSamples, density, true, trial_ctr, s, [](RunShape) { return true; },
+    const int ng = build_groups(kv, gshift, hlist, nh, cwork, tmp, rd, s, err);
+    (void)hipEventRecord(e0, s);
+    if (ng > 0) {
+        const RunShape sh = tuned_run_launch(
+            prec, kRunSamples, (double)nh / ng, false, trial_ctr, s,
+            [&](RunShape c) {
+                nr = build_run_starts(g, kv, gshift, hlist, nh, ng, c.kx, cwork, tmp, &rstart, rd, s, err);
+                return nr > 0;
+            },
             [&](RunShape c, bool trial) {
-                launch_wave_samples(prec, c.T, g, ra, rg, fc, lv, list, kv, hlist, nh, vals, ent,
-                                    trial ? trial_ctr : ctr, s);
+                launch_run_samples(prec, c.T, g, ra, rg, fc, lv, list, kv, hlist, rstart, vals, nr, ent,
+                                   trial ? trial_ctr : ctr, s);
             });
-        nr = (nh + kWave - 1) / kWave;
-    } else {
-        const int ng = build_groups(kv, gshift, hlist, nh, cwork, tmp, rd, s, err);
-        (void)hipEventRecord(e0, s);
-        if (ng > 0) {
-            const RunShape sh = tuned_run_launch(
-                prec, kRunSamples, (double)nh / ng, false, trial_ctr, s,
-                [&](RunShape c) {
-                    nr = build_run_starts(g, kv, gshift, hlist, nh, ng, c.kx, cwork, tmp, &rstart, rd, s, err);
-                    return nr > 0;
-                },
-                [&](RunShape c, bool trial) {
-                    launch_run_samples(prec, c.T, g, ra, rg, fc, lv, list, kv, hlist, rstart, vals, nr, ent,
-                                       trial ? trial_ctr : ctr, s);
-                });
-            *kx_out = sh.kx;
-        }
+        *kx_out = sh.kx;
     }
     *nruns_out = nr;
     (void)hipEventRecord(e1, s);

@@ -209,12 +209,21 @@ void launch_sample_dedupe_keys(GridDev g, NodeLevel lv, const int* list, int64_t
 // and point (rent: node * 27 + sample; the level's node count times 27 must fit an int)
 void launch_sample_tiles(GridDev g, NodeLevel lv, const int* list, int64_t k, const float origin[3], int lb,
                          int vbits, int* nrec, int* ent_rec, uint64_t* rkey, int* rval, int* rent, hipStream_t s);
+// The k listed nodes' samples merged per tile, evaluated between events e0 / e1 and written to the level's samples,
+// without a sort or a read-back: nrec (1 int), ent_rec (27 k ints), rent and vals (tile_record_bound(k)
+// ints and values, the bound and the level's node count times 27 below 2^31) are work space
+inline int64_t tile_record_bound(int64_t k) { return 27 * k + 64 * ((k + 255) / 256); }
+bool samples_by_tile(int64_t k, double density);  // the rule: density in sample points per hash cell
+void launch_samples_by_tile(int prec, GridDev g, const void* rec_a, const void* rec_g, FieldConst fc, NodeLevel lv,
+                            const int* list, int64_t k, double density, int* nrec, int* ent_rec, int* rent, void* vals,
+                            void* samples, Counters* ctr, Counters* trial_ctr, hipEvent_t e0, hipEvent_t e1,
+                            hipStream_t s);
 // Distinct points of nrec sorted items evaluated and their values scattered to the level's samples.
 // ent NULL: the items are the sample entries (nent == nrec, ent_rec and rec_head unused); else
 // item value v is a record slot, ent[v] its node * 27 + sample, ent_rec the record slot of each of
 // nent entries and rec_head (one int per slot) scratch.
 void launch_sample_dedupe_eval(int prec, GridDev g, const void* rec_a, const void* rec_g, FieldConst fc, NodeLevel lv,
-                               const int* list, SortedKV kv, const int* ent, int gshift, double density, int64_t nrec,
+                               const int* list, SortedKV kv, const int* ent, int gshift, int64_t nrec,
                                const int* ent_rec, int64_t nent, int* rec_head, int* head, int* hpos, int* rep,
                                int* hlist, int* cwork, int64_t* nheads_out, int64_t* nruns_out, int* kx_out,
                                void* vals, void* samples, int* tmp, Counters* ctr, Counters* trial_ctr, hipEvent_t e0,

@@ -26,15 +26,13 @@ struct RunShape {
     int kx;  // cells per run, or 0: 64 consecutive points per wave (wave_eval.h)
 };
 
-// Points of a lattice with at least kWaveDensity points per hash cell, and at least kWaveMin of them, go 64 to a
-// wave (wave_eval.h) and no runs are built. The octree's levels hold 64 (deepest sampled, leaf centres), 8 and 1
+// Points of a lattice with at least kWaveDensity points per hash cell go 64 to a wave (wave_eval.h) and no runs are
+// built (leaf centres: from kWaveMin on). The octree's levels hold 64 or more (deepest sampled, leaf centres), 8 and 1
 // points per cell, level by level upwards. At 64 and 8 a wave's points share a few cells, so one test of all of
 // them against the union of their windows beats each thread testing its own window: crown splash, 4 M
 // particles, compensated FP32, 11.9 M + 2.4 M points: 1.65 ms against 2.05 ms as runs, centres 0.46 against
 // 0.57 ms. At 1 a wave spans five row pieces and tests 18 candidates for each one in a point's
-// window: 0.70 ms against 0.52 ms for D_min's 1.05 M points. A launch of few points lasts as long as its
-// slowest wave, and a wave of 64 points in several rows is slower than a small run: a 14 k-particle frame's
-// 120 k points took 128 us against 53 us; above 2^18 points both kinds fill the chip.
+// window: 0.70 ms against 0.52 ms for D_min's 1.05 M points.
 constexpr double kWaveDensity = 4.0;
 constexpr int64_t kWaveMin = 1 << 18;
 

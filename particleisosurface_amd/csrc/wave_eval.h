@@ -124,10 +124,11 @@ __device__ __forceinline__ void wave_cull(const float4* cull, const WavePoints& 
 }
 
 // Adds to st the contributions of the candidates of point p (act: the lane has a point) and returns
-// their number, passing or not. Every lane of the wave calls it. SORTED: the points come in
-// cell order, active lanes first; otherwise any order is right, and neighbouring lanes should lie
-// close together.
-template <bool SORTED, class Pol>
+// their number, passing or not. Every lane of the wave calls it. Neighbouring lanes should lie close
+// together; any order is right unless kWaveSorted is given, which says that the points come in cell order,
+// active lanes first. BACK: cells before the first lane's that its row piece may take.
+constexpr int kWaveSorted = -1;
+template <int BACK, class Pol>
 __device__ __forceinline__ int wave_visit(const GridDev& g, const Pol& pol, typename Pol::State& st, bool act,
                                           const float p[3], WaveLds<Pol>& L) {
     typedef typename Pol::Real Real;
@@ -144,7 +145,8 @@ __device__ __forceinline__ int wave_visit(const GridDev& g, const Pol& pol, type
         const int lx = __builtin_amdgcn_readlane(ix, lead), ly = __builtin_amdgcn_readlane(iy, lead),
                   lz = __builtin_amdgcn_readlane(iz, lead);
         // the lanes taken with the leader: its row, and at most kWaveCells cells
-        constexpr int kBack = SORTED ? 0 : kWaveCells / 2;
+        constexpr bool SORTED = BACK == kWaveSorted;
+        constexpr int kBack = SORTED ? 0 : BACK;
         const bool mem = ((rem >> lane) & 1) && iy == ly && iz == lz && (unsigned)(ix - lx + kBack) < (unsigned)kWaveCells;
         const unsigned long long mm = __ballot(mem);
         rem &= ~mm;
@@ -384,18 +386,17 @@ template <class R, bool K, bool GRAD, int MODE> struct WaveField {
     }
 };
 
-// Points h = blockIdx.x * T + threadIdx.x < n of src (in cell order) evaluated by the waves of a block of T
-// threads; returns the candidates of this thread's point.
-template <int T, class R, bool K, bool GRAD, int MODE, class Src>
+// Points h = blockIdx.x * T + threadIdx.x < n of src evaluated by the waves of a block of T threads; returns the
+// candidates of this thread's point. bool src.point(h, p) gives a point or says that there is none.
+template <int T, class R, bool K, bool GRAD, int MODE, int BACK = kWaveSorted, class Src>
 __device__ __forceinline__ int wave_eval(const GridDev& g, const Recs<R>& rec, const FieldConst& fc, const Src& src,
                                          int n, WaveLds<WaveField<R, K, GRAD, MODE>>* lds) {
     const WaveField<R, K, GRAD, MODE> pol(rec, fc);
     const int h = (int)blockIdx.x * T + (int)threadIdx.x;
-    const bool act = h < n;
     float p[3] = {0.f, 0.f, 0.f};
-    if (act) src.point(h, p);
+    const bool act = h < n && src.point(h, p);
     typename WaveField<R, K, GRAD, MODE>::State st{R(p[0]), R(p[1]), R(p[2])};
-    const int ncand = wave_visit<true>(g, pol, st, act, p, lds[threadIdx.x / kWave]);
+    const int ncand = wave_visit<BACK>(g, pol, st, act, p, lds[threadIdx.x / kWave]);
     if (act) {
         const R gr[3] = {st.ga[0].get(), st.ga[1].get(), st.ga[2].get()};
         src.store(h, st.acc.get(), gr);
