@@ -798,15 +798,22 @@ int sweep(pisurf_ctx* c, LevelBuf* L, int32_t* sc_dev, int level_depth) {
     // Deduplicated sampling needs one node size per level (lattice keys) and 21-bit lattice
     // coordinates: 2^(depth + 1) half-widths span the root box.
     // levels above D_min sample nothing (wants_samples), so they skip the count read-back
-    const bool dedupe = c->prm.sample_dedupe && level_depth >= 0 && level_depth <= 19 && level_depth >= c->dmin;
+    // and the leaf-depth level samples nothing unless the QEF does
+    const bool dedupes = c->prm.sample_dedupe && level_depth >= 0 && level_depth <= 19;
+    const bool no_samples = dedupes && leaf_level && c->prm.qef_mode == 0;
+    const bool dedupe = dedupes && !no_samples && level_depth >= c->dmin;
     // centre values of the leaf-depth level by runs (QEF off); that count is read after the
     // sampling's reads, so it is published far from the bytes they copy
     const bool centre_runs = level_depth >= 0 && leaf_level && c->prm.qef_mode == 0 && level_depth >= c->dmin;
     const ScanPub kpub = dedupe ? c->scan_pub() : ScanPub();
     const ScanPub cpub = centre_runs ? c->scan_pub(kScanPubFar) : ScanPub();
-    launch_sample_list(tp, v, L->flag.as<int>(), L->scanned.as<int>(), L->child.as<int>(), c->cl_flag.as<int>(),
-                       c->cl_pos.as<int>(), c->cl_list.as<int>(), c->tmp.as<int>(), c->stream, kpub, cpub);
-    if (dedupe) {
+    HIPCHK(c, c->sd_nrec.ensure(4));
+    launch_sample_list(tp, v, no_samples ? nullptr : L->flag.as<int>(), L->scanned.as<int>(), L->child.as<int>(),
+                       level_depth < 0 || centre_runs ? c->cl_flag.as<int>() : nullptr, c->cl_pos.as<int>(),
+                       c->cl_list.as<int>(), c->sd_nrec.as<int>(), c->tmp.as<int>(), c->stream, kpub, cpub);
+    if (no_samples) {
+        // leaf-depth nodes, whose centres follow
+    } else if (dedupe) {
         int k = 0;
         HIPCHK(c, c->read_scan(&k, L->scanned.as<int>() + L->n, kpub));
         const int64_t nent = (int64_t)k * 27;
@@ -819,7 +826,6 @@ int sweep(pisurf_ctx* c, LevelBuf* L, int32_t* sc_dev, int level_depth) {
             const bool tiles = L->n * 27 < INT32_MAX;
             const double density = lattice_density(c, level_depth, 2);
             if (tiles && samples_by_tile(k, density)) {
-                HIPCHK(c, c->sd_nrec.ensure(4));
                 HIPCHK(c, c->sd_entrec.ensure(nent * 4));
                 HIPCHK(c, c->sd_rent.ensure(tile_record_bound(k) * 4));
                 HIPCHK(c, c->sd_vals.ensure(tile_record_bound(k) * rsz));
@@ -837,7 +843,6 @@ int sweep(pisurf_ctx* c, LevelBuf* L, int32_t* sc_dev, int level_depth) {
                     HIPCHK(c, c->sd_entrec.ensure(nent * 4));
                     HIPCHK(c, c->sd_rent.ensure(nent * 4));
                     HIPCHK(c, c->sd_rechead.ensure(nent * 4));
-                    HIPCHK(c, c->sd_nrec.ensure(4));
                 }
                 HIPCHK(c, c->sd_head.ensure((2 * ((nent + 255) / 256) + 2) * 4));
                 HIPCHK(c, c->sd_hpos.ensure((nent + 1) * 4));
@@ -1820,7 +1825,7 @@ int batch_level_begin(BatchFrame& f, BatchReads& br) {
     HIPCHK(c, c->cl_pos.ensure((L->n + 1) * 4));
     HIPCHK(c, c->cl_list.ensure((L->n + 1) * 4));
     launch_sample_list(f.tp, v, L->flag.as<int>(), L->scanned.as<int>(), L->child.as<int>(), c->cl_flag.as<int>(),
-                       c->cl_pos.as<int>(), c->cl_list.as<int>(), c->tmp.as<int>(), c->stream);
+                       c->cl_pos.as<int>(), c->cl_list.as<int>(), nullptr, c->tmp.as<int>(), c->stream);
     f.dedupe = c->prm.sample_dedupe && ld <= 19 && ld >= c->dmin;
     f.centers = f.leaf_level && c->prm.qef_mode == 0 && ld >= c->dmin;
     f.ksamp = f.kcent = f.nh = f.ng = f.nr = f.ngc = f.nrc = 0;

@@ -5,6 +5,7 @@
 #include <cstring>
 #include <mutex>
 #include <new>
+#include <type_traits>
 #include <vector>
 
 #include "pisurf_internal.h"
@@ -98,6 +99,37 @@ __global__ void __launch_bounds__(kScanT) k_scan_add_prefix(int* __restrict__ ou
     }
 }
 
+// Up to kScanOne elements by one workgroup: two launches of a few microseconds each become one.
+constexpr int kOneT = 1024, kOneI = 16;
+constexpr int64_t kScanOne = kOneT * kOneI;
+__global__ void __launch_bounds__(kOneT) k_scan_one(const int* __restrict__ in, int* __restrict__ out, int n, char* pdst,
+                                                    int poff, uint32_t pseq) {
+    __shared__ int wsum[kOneT / kWave];
+    const int t = threadIdx.x, lane = t & 63, w = t >> 6;
+    const int per = (n + kOneT - 1) / kOneT, base = t * per;  // consecutive elements of this thread
+    int v[kOneI];
+    int acc = 0;
+#pragma unroll
+    for (int k = 0; k < kOneI; k++) {
+        v[k] = (k < per && base + k < n) ? in[base + k] : 0;
+        acc += v[k];
+    }
+    const int incl = wave_incl_scan(acc, lane);
+    if (lane == kWave - 1) wsum[w] = incl;
+    __syncthreads();
+    int s = lane < kOneT / kWave ? wsum[lane] : 0;
+    s = wave_incl_scan(s, lane);
+    int run = incl - acc + (w > 0 ? __shfl(s, w - 1, kWave) : 0);
+#pragma unroll
+    for (int k = 0; k < kOneI; k++) {
+        if (k < per && base + k < n) {
+            out[base + k] = run;
+            if (pdst && base + k == n - 1) scan_publish(pdst, poff, pseq, run);
+        }
+        run += v[k];
+    }
+}
+
 int64_t scan_tmp_ints(int64_t n) {
     int64_t tot = 0;
     while (n > 1) {
@@ -110,6 +142,10 @@ int64_t scan_tmp_ints(int64_t n) {
 void exclusive_scan_i32(const int* in, int* out, int64_t n, int* tmp, hipStream_t s, ScanPub pub) {
     if (n <= 0) return;
     const int64_t nb = (n + kScanTile - 1) / kScanTile;
+    if (nb > 1 && n <= kScanOne) {
+        k_scan_one<<<1, kOneT, 0, s>>>(in, out, (int)n, pub.dst, pub.off, pub.seq);
+        return;
+    }
     int* sums = tmp;
     int* sums_scanned = tmp + nb + 1;
     k_scan_tile<<<dim3((unsigned)nb), dim3(kScanT), 0, s>>>(in, out, n, sums, nb == 1 ? pub.dst : nullptr, pub.off,
@@ -131,9 +167,22 @@ void exclusive_scan_i32(const int* in, int* out, int64_t n, int* tmp, hipStream_
 // ---------------------------------------------------------------------------------------------
 constexpr int kRsT = 256, kRsRounds = 16, kRsTile = kRsT * kRsRounds, kRsDigits = 256;
 
+// How the tiles' digit counts become each tile's first output position per digit:
+//   kRsSelf  up to kRsSelfTiles tiles (262 k keys): counts tile by tile; the scatter adds them up itself (64 KB
+//            of reads per workgroup at most), so a pass is two launches
+//   kRsTiled up to kRsSumTiles tiles (8 M keys): counts digit-major, scanned in pieces of kScanTile; the scatter adds
+//            the piece's offset, from the pieces' totals (one per thread): three launches
+//   kRsFull  more: counts digit-major, scanned completely
+// A frame waits for each launch where its kernels take 2 - 5 us. With these passes, kScanOne and one list per level
+// a 14 k-particle frame takes 1.38 ms instead of 1.42, 400 k particles in FP64 3.04 instead of 3.10, 4 M 11.86
+// instead of 11.97.
+enum { kRsSelf = 0, kRsTiled = 1, kRsFull = 2 };
+constexpr int kRsSelfTiles = 64;
+constexpr int kRsSumTiles = kScanTile / kRsDigits * kRsT;
+
 template <class KT>
 __global__ void __launch_bounds__(kRsT) k_rs_hist(const KT* __restrict__ keys, int64_t n, int shift,
-                                                  int* __restrict__ bh, int nblocks) {
+                                                  int* __restrict__ bh, int nblocks, int mode) {
     __shared__ int h[4][kRsDigits];  // one histogram per wave: atomics of different waves do not collide
     const int t = threadIdx.x, w = t >> 6;
     h[0][t] = h[1][t] = h[2][t] = h[3][t] = 0;
@@ -145,7 +194,8 @@ __global__ void __launch_bounds__(kRsT) k_rs_hist(const KT* __restrict__ keys, i
         if (i < n) atomicAdd(&h[w][(int)((keys[i] >> shift) & 255u)], 1);
     }
     __syncthreads();
-    bh[(int64_t)t * nblocks + blockIdx.x] = h[0][t] + h[1][t] + h[2][t] + h[3][t];
+    const int64_t at = mode == kRsSelf ? (int64_t)blockIdx.x * kRsDigits + t : (int64_t)t * nblocks + blockIdx.x;
+    bh[at] = h[0][t] + h[1][t] + h[2][t] + h[3][t];
 }
 
 // Scatter of one tile: wave w takes the tile's keys [w * 1024, (w + 1) * 1024) in 16 rounds of 64.
@@ -155,11 +205,13 @@ __global__ void __launch_bounds__(kRsT) k_rs_hist(const KT* __restrict__ keys, i
 // in the tile sorted by digit (thread t owns consecutive digits); the tile is staged in LDS in
 // that order and written out by consecutive threads, so each digit's run of keys goes to
 // consecutive addresses.
-template <class KT, bool VAL>
+template <class KT, bool VAL, int MODE>
 __global__ void __launch_bounds__(kRsT) k_rs_scatter(const KT* __restrict__ kin, const int* __restrict__ vin,
                                                      KT* __restrict__ kout, int* __restrict__ vout, int64_t n,
-                                                     int shift, const int* __restrict__ bscan, int nblocks) {
+                                                     int shift, const int* __restrict__ bscan,
+                                                     const int* __restrict__ sums, int nblocks) {
     constexpr int DB = 8, ND = 1 << DB, DPT = ND / kRsT;
+    static_assert(ND == kRsT, "a thread per digit");
     __shared__ int base[ND];
     __shared__ int cnt[4][ND];
     __shared__ int dstart[ND];
@@ -167,9 +219,36 @@ __global__ void __launch_bounds__(kRsT) k_rs_scatter(const KT* __restrict__ kin,
     __shared__ KT sk[kRsTile];
     __shared__ int sv[VAL ? kRsTile : 1];
     const int t = threadIdx.x, w = t >> 6, lane = t & 63;
-    for (int d = t; d < ND; d += kRsT) {
-        base[d] = bscan[(int64_t)d * nblocks + blockIdx.x];
-        cnt[0][d] = cnt[1][d] = cnt[2][d] = cnt[3][d] = 0;
+    cnt[0][t] = cnt[1][t] = cnt[2][t] = cnt[3][t] = 0;
+    if (MODE == kRsFull) {
+        base[t] = bscan[(int64_t)t * nblocks + blockIdx.x];
+    } else {
+        // exclusive sums over the workgroup: of the digits' totals, or of the scan pieces' totals
+        int mine = 0, before = 0;
+        if (MODE == kRsSelf) {
+#pragma unroll 8
+            for (int b = 0; b < nblocks; b++) {
+                const int v = bscan[b * ND + t];
+                mine += v;
+                before += b < (int)blockIdx.x ? v : 0;
+            }
+        } else {
+            const int pieces = (int)(((int64_t)ND * nblocks + kScanTile - 1) / kScanTile);
+            mine = t < pieces ? sums[t] : 0;
+        }
+        const int inc = wave_incl_scan(mine, lane);
+        if (lane == kWave - 1) wsum[w] = inc;
+        __syncthreads();
+        int ex = inc - mine;
+        for (int ww = 0; ww < w; ww++) ex += wsum[ww];
+        if (MODE == kRsSelf) {
+            base[t] = ex + before;
+        } else {
+            dstart[t] = ex;  // (dstart is filled later)
+            __syncthreads();
+            const int64_t at = (int64_t)t * nblocks + blockIdx.x;
+            base[t] = bscan[at] + dstart[at / kScanTile];
+        }
     }
     __syncthreads();
     const unsigned long long lt = (lane == 0) ? 0ull : ((~0ull) >> (64 - lane));
@@ -258,12 +337,23 @@ static KT* radix_passes(KT* k0, int* v0, KT* k1, int* v1, int64_t n, int lo_bit,
     const int passes = (bits + 7) / 8;
     KT *ks = k0, *kd = k1;
     int *vs = v0, *vd = v1;
+    const int mode = nb <= kRsSelfTiles ? kRsSelf : nb <= kRsSumTiles ? kRsTiled : kRsFull;
+    const int64_t nc = kRsDigits * (int64_t)nb;
     for (int p = 0; p < passes; p++) {
         const int shift = lo_bit + 8 * p;
-        k_rs_hist<KT><<<nb, kRsT, 0, s>>>(ks, n, shift, bh, nb);
-        exclusive_scan_i32(bh, bscan, kRsDigits * (int64_t)nb, stmp, s);
-        if (vs) k_rs_scatter<KT, true><<<nb, kRsT, 0, s>>>(ks, vs, kd, vd, n, shift, bscan, nb);
-        else k_rs_scatter<KT, false><<<nb, kRsT, 0, s>>>(ks, nullptr, kd, nullptr, n, shift, bscan, nb);
+        k_rs_hist<KT><<<nb, kRsT, 0, s>>>(ks, n, shift, bh, nb, mode);
+        if (mode == kRsFull) exclusive_scan_i32(bh, bscan, nc, stmp, s);
+        if (mode == kRsTiled)
+            k_scan_tile<<<(unsigned)((nc + kScanTile - 1) / kScanTile), kScanT, 0, s>>>(bh, bscan, nc, stmp, nullptr, 0, 0);
+        auto scatter = [&](auto m) {
+            constexpr int M = decltype(m)::value;
+            const int* b = M == kRsSelf ? bh : bscan;
+            if (vs) k_rs_scatter<KT, true, M><<<nb, kRsT, 0, s>>>(ks, vs, kd, vd, n, shift, b, stmp, nb);
+            else k_rs_scatter<KT, false, M><<<nb, kRsT, 0, s>>>(ks, nullptr, kd, nullptr, n, shift, b, stmp, nb);
+        };
+        if (mode == kRsSelf) scatter(std::integral_constant<int, kRsSelf>());
+        else if (mode == kRsTiled) scatter(std::integral_constant<int, kRsTiled>());
+        else scatter(std::integral_constant<int, kRsFull>());
         KT* tk = ks; ks = kd; kd = tk;
         int* tv = vs; vs = vd; vd = tv;
     }

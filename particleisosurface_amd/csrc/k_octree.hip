@@ -176,11 +176,9 @@ __global__ void __launch_bounds__(256) k_empty_curv(GridDev g, const float4* __r
 // 27 samples, or only its centre value (stored in sample slot 13) when it sits at leaf depth.
 __global__ void k_sample_flag(TreeParams tp, NodeLevel lv, int* __restrict__ flag, int* __restrict__ cflag) {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < lv.n) {
-        flag[i] = wants_samples(lv, tp, i) ? 1 : 0;
-        cflag[i] = wants_center(lv, tp, i) ? 1 : 0;
-    }
-    if (i == lv.n) flag[i] = cflag[i] = 0;
+    if (i > lv.n) return;
+    if (flag) flag[i] = i < lv.n && wants_samples(lv, tp, i) ? 1 : 0;
+    if (cflag) cflag[i] = i < lv.n && wants_center(lv, tp, i) ? 1 : 0;
 }
 
 // ---- per-level sample deduplication --------------------------------------------------------
@@ -732,7 +730,6 @@ __global__ void k_entry_scatter(const int* __restrict__ list, const int* __restr
 
 void launch_sample_tiles(GridDev g, NodeLevel lv, const int* list, int64_t k, const float origin[3], int lb,
                          int vbits, int* nrec, int* ent_rec, uint64_t* rkey, int* rval, int* rent, hipStream_t s) {
-    launch_fill_i32(nrec, 1, 0, s);
     if (k > 0)
         k_sample_tiles<false><<<(unsigned)((k + kStT - 1) / kStT), kStT, 0, s>>>(
             g, lv, list, k, origin[0], origin[1], origin[2], lb, vbits, nrec, ent_rec, rkey, rval, rent);
@@ -872,8 +869,9 @@ __global__ void __launch_bounds__(256) k_centers(GridDev g, Recs<R> rec, FieldCo
     wave_count(&ctr_stripe(ctr)->candidates, (unsigned long long)vis);
 }
 __global__ void k_sample_list(NodeLevel lv, const int* __restrict__ flag, const int* __restrict__ pos,
-                              int* __restrict__ list) {
+                              int* __restrict__ list, int* __restrict__ zero) {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (zero && i == 0) *zero = 0;
     if (i < lv.n && flag[i]) list[pos[i]] = (int)i;
 }
 
@@ -1205,13 +1203,17 @@ void launch_empty_curv(GridDev g, const float4* spos, const float4* nrm, TreePar
 }
 
 void launch_sample_list(TreeParams tp, NodeLevel lv, int* flag, int* pos, int* list, int* cflag, int* cpos,
-                        int* clist, int* tmp, hipStream_t s, ScanPub pub, ScanPub cpub) {
+                        int* clist, int* zero, int* tmp, hipStream_t s, ScanPub pub, ScanPub cpub) {
     if (lv.n <= 0) return;
     k_sample_flag<<<(unsigned)((lv.n + 1 + 255) / 256), 256, 0, s>>>(tp, lv, flag, cflag);
-    exclusive_scan_i32(flag, pos, lv.n + 1, tmp, s, pub);
-    k_sample_list<<<(unsigned)((lv.n + 255) / 256), 256, 0, s>>>(lv, flag, pos, list);
-    exclusive_scan_i32(cflag, cpos, lv.n + 1, tmp, s, cpub);
-    k_sample_list<<<(unsigned)((lv.n + 255) / 256), 256, 0, s>>>(lv, cflag, cpos, clist);
+    if (flag) {
+        exclusive_scan_i32(flag, pos, lv.n + 1, tmp, s, pub);
+        k_sample_list<<<(unsigned)((lv.n + 255) / 256), 256, 0, s>>>(lv, flag, pos, list, zero);
+    }
+    if (cflag) {
+        exclusive_scan_i32(cflag, cpos, lv.n + 1, tmp, s, cpub);
+        k_sample_list<<<(unsigned)((lv.n + 255) / 256), 256, 0, s>>>(lv, cflag, cpos, clist, nullptr);
+    }
 }
 
 void launch_sample_dedupe_keys(GridDev g, NodeLevel lv, const int* list, int64_t nent, const float origin[3],
@@ -1266,7 +1268,6 @@ void launch_samples_by_tile(int prec, GridDev g, const void* ra, const void* rg,
                             void* samples, Counters* ctr, Counters* trial_ctr, hipEvent_t e0, hipEvent_t e1,
                             hipStream_t s) {
     const unsigned tiles = (unsigned)((k + kStT - 1) / kStT);
-    launch_fill_i32(nrec, 1, 0, s);
     k_sample_tiles<true><<<tiles, kStT, 0, s>>>(g, lv, list, k, 0.f, 0.f, 0.f, 0, 0, nrec, ent_rec, nullptr, nullptr,
                                                 rent);
     const int64_t most = tile_record_bound(k);

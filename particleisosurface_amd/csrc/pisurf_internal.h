@@ -183,9 +183,11 @@ void launch_empty_curv(GridDev g, const float4* spos, const float4* nrm, TreePar
                        int pass, const void* samples, int rsz, hipStream_t s);
 // flag[n+1], pos[n+1] (pos[n] = number of listed nodes, published to pub), list[n]: nodes to
 // sample; cflag / cpos / clist: leaf-depth nodes that need only their centre value (cpos[n]
-// published to cpub)
+// published to cpub). flag or cflag NULL: the caller knows that the level has no such nodes. zero
+// (may be NULL): a counter cleared along with the first list
 void launch_sample_list(TreeParams tp, NodeLevel lv, int* flag, int* pos, int* list, int* cflag, int* cpos,
-                        int* clist, int* tmp, hipStream_t s, ScanPub pub = ScanPub(), ScanPub cpub = ScanPub());
+                        int* clist, int* zero, int* tmp, hipStream_t s, ScanPub pub = ScanPub(),
+                        ScanPub cpub = ScanPub());
 void launch_centers(int prec, GridDev g, const void* rec_a, const void* rec_g, FieldConst fc, NodeLevel lv,
                     const int* list, const int* count, void* samples, Counters* ctr, hipStream_t s);
 // the same for k listed centres (count known on the host), grouped by hash cell and evaluated in
@@ -203,14 +205,14 @@ void launch_centers_runs(int prec, GridDev g, const void* rec_a, const void* rec
 // number of cells of a row per run. Counts are read back through rd; a failed read sets *err.
 void launch_sample_dedupe_keys(GridDev g, NodeLevel lv, const int* list, int64_t nent, const float origin[3],
                                int lb, int vbits, uint64_t* key, int* val, hipStream_t s);
-// Sample records merged per tile of 256 listed nodes: the record count in *nrec (cleared here),
+// Sample records merged per tile of 256 listed nodes: the record count in *nrec (cleared by launch_sample_list),
 // every entry's record slot (ent_rec, < k * 27), per record its sort key as
 // launch_sample_dedupe_keys makes it (packed with the slot when vbits > 0, else the slot in rval)
 // and point (rent: node * 27 + sample; the level's node count times 27 must fit an int)
 void launch_sample_tiles(GridDev g, NodeLevel lv, const int* list, int64_t k, const float origin[3], int lb,
                          int vbits, int* nrec, int* ent_rec, uint64_t* rkey, int* rval, int* rent, hipStream_t s);
 // The k listed nodes' samples merged per tile, evaluated between events e0 / e1 and written to the level's samples,
-// without a sort or a read-back: nrec (1 int), ent_rec (27 k ints), rent and vals (tile_record_bound(k)
+// without a sort or a read-back: nrec (1 int, cleared by launch_sample_list), ent_rec (27 k ints), rent and vals (tile_record_bound(k)
 // ints and values, the bound and the level's node count times 27 below 2^31) are work space
 inline int64_t tile_record_bound(int64_t k) { return 27 * k + 64 * ((k + 255) / 256); }
 bool samples_by_tile(int64_t k, double density);  // the rule: density in sample points per hash cell
