@@ -46,6 +46,21 @@ __device__ __forceinline__ bool wants_center(const NodeLevel& lv, const TreePara
            lv.depth[node] >= tp.depth_min;
 }
 
+// the node's 27 samples do not all have the same sign
+__device__ __forceinline__ bool signs_differ(const void* samples, int rsz, int64_t node) {
+    bool sc = false;
+    if (rsz == 8) {
+        const double* f = (const double*)samples + node * 27;
+        const bool s0 = f[0] >= 0.0;
+        for (int k = 1; k < 27; k++) sc = sc || ((f[k] >= 0.0) != s0);
+    } else {
+        const float* f = (const float*)samples + node * 27;
+        const bool s0 = f[0] >= 0.0f;
+        for (int k = 1; k < 27; k++) sc = sc || ((f[k] >= 0.0f) != s0);
+    }
+    return sc;
+}
+
 template <int G, int PASS>
 __global__ void __launch_bounds__(256) k_empty_curv(GridDev g, const float4* __restrict__ spos,
                                                     const float4* __restrict__ nrm, TreeParams tp, NodeLevel lv,
@@ -58,17 +73,7 @@ __global__ void __launch_bounds__(256) k_empty_curv(GridDev g, const float4* __r
         // classification reads curv only for sampled nodes whose samples change sign (the exits
         // below are uniform over the node's lanes)
         if (!tp.curv || !wants_samples(lv, tp, node)) return;
-        bool sc = false;
-        if (rsz == 8) {
-            const double* f = (const double*)samples + node * 27;
-            const bool s0 = f[0] >= 0.0;
-            for (int k = 1; k < 27; k++) sc = sc || ((f[k] >= 0.0) != s0);
-        } else {
-            const float* f = (const float*)samples + node * 27;
-            const bool s0 = f[0] >= 0.0f;
-            for (int k = 1; k < 27; k++) sc = sc || ((f[k] >= 0.0f) != s0);
-        }
-        if (!sc) return;
+        if (!signs_differ(samples, rsz, node)) return;
         if (!tp.calc_normals) {  // no normals: curv = 1 (no normal length)
             if (lane == 0) lv.curv[node] = 1.0f;
             return;
@@ -171,6 +176,32 @@ __global__ void __launch_bounds__(256) k_empty_curv(GridDev g, const float4* __r
     }
 }
 
+
+// mark[cell] = 1 for the cells whose particles' normals a curvature below this level can read: those of the grown
+// boxes (k_empty_curv) of the sampled nodes whose samples change sign, which hold the grown boxes of all
+// their descendants; slack covers the rounding of the descendants' coordinates. A group of 16 lanes per node.
+__global__ void __launch_bounds__(256) k_mark_cells(GridDev g, TreeParams tp, NodeLevel lv,
+                                                    const void* __restrict__ samples, int rsz, float slack,
+                                                    uint8_t* __restrict__ mark) {
+    const int64_t node = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) / 16;
+    const int lane = threadIdx.x % 16;
+    if (node >= lv_count(lv) || !wants_samples(lv, tp, node) || !signs_differ(samples, rsz, node)) return;
+    const float4 c = lv.c[node];
+    const float cc[3] = {c.x, c.y, c.z};
+    int lo[3], hi[3];
+#pragma unroll
+    for (int a = 0; a < 3; a++) {
+        const float grow = c.w + tp.margin + slack;
+        lo[a] = max(0, cell_coord(cc[a] - grow, g.b0[a], g.cell, g.n[a]));
+        hi[a] = min(g.n[a] - 1, cell_coord(cc[a] + grow, g.b0[a], g.cell, g.n[a]));
+    }
+    const int ny = hi[1] - lo[1] + 1, nz = hi[2] - lo[2] + 1;
+    if (ny <= 0 || nz <= 0) return;
+    for (int row = lane; row < ny * nz; row += 16) {
+        const int64_t base = ((int64_t)(lo[2] + row / ny) * g.n[1] + lo[1] + row % ny) * g.n[0];
+        for (int x = lo[0]; x <= hi[0]; x++) mark[base + x] = 1;
+    }
+}
 
 // compaction of the nodes to evaluate: flag, then (after a scan) the list. A listed node gets its
 // 27 samples, or only its centre value (stored in sample slot 13) when it sits at leaf depth.
@@ -1200,6 +1231,12 @@ void launch_empty_curv(GridDev g, const float4* spos, const float4* nrm, TreePar
     if (pass == kEmptyOnly) go(std::integral_constant<int, kEmptyOnly>());
     else if (pass == kCurvOnly) go(std::integral_constant<int, kCurvOnly>());
     else go(std::integral_constant<int, kEmptyAndCurv>());
+}
+
+void launch_mark_cells(GridDev g, TreeParams tp, NodeLevel lv, const void* samples, int rsz, float slack, uint8_t* mark,
+                       hipStream_t s) {
+    if (lv.n <= 0) return;
+    k_mark_cells<<<(unsigned)((lv.n + 15) / 16), 256, 0, s>>>(g, tp, lv, samples, rsz, slack, mark);
 }
 
 void launch_sample_list(TreeParams tp, NodeLevel lv, int* flag, int* pos, int* list, int* cflag, int* cpos,

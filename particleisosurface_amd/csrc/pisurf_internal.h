@@ -136,9 +136,10 @@ bool eval_points_sorts(int64_t n, int64_t particles);
 void launch_eval_points_sorted(int prec, GridDev g, const void* rec_a, const void* rec_g, FieldConst fc, const float* q,
                                int64_t n, double* f, double* grad, uint64_t* key, int* val, uint64_t* key2, int* val2,
                                int* tmp, Counters* ctr, hipStream_t s);
-// trial_ctr: counter block for the timed trial launches of shape tuning (their counts are not kept)
+// mark (may be NULL): only the runs with a marked cell. trial_ctr: counter block for the timed trial launches of shape
+// tuning (their counts are not kept)
 void launch_normals(int prec, GridDev g, const void* rec_a, const void* rec_g, FieldConst fc, const float4* spos,
-                    int64_t n, int64_t n_invalid, float4* nrm, Counters* ctr, Counters* trial_ctr, hipStream_t s);
+                    int64_t n, int64_t n_invalid, const uint8_t* mark, float4* nrm, Counters* ctr, Counters* trial_ctr, hipStream_t s);
 // dense sampling box: lo / hi corners, steps (intervals) and dims = steps + 1 points per axis
 struct UniformBox {
     float lo[3], hi[3];
@@ -188,6 +189,8 @@ void launch_empty_curv(GridDev g, const float4* spos, const float4* nrm, TreePar
 void launch_sample_list(TreeParams tp, NodeLevel lv, int* flag, int* pos, int* list, int* cflag, int* cpos,
                         int* clist, int* zero, int* tmp, hipStream_t s, ScanPub pub = ScanPub(),
                         ScanPub cpub = ScanPub());
+void launch_mark_cells(GridDev g, TreeParams tp, NodeLevel lv, const void* samples, int rsz, float slack, uint8_t* mark,
+                       hipStream_t s);
 void launch_centers(int prec, GridDev g, const void* rec_a, const void* rec_g, FieldConst fc, NodeLevel lv,
                     const int* list, const int* count, void* samples, Counters* ctr, hipStream_t s);
 // the same for k listed centres (count known on the host), grouped by hash cell and evaluated in

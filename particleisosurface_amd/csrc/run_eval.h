@@ -238,12 +238,13 @@ inline int cell_group_bits(const GridDev& g) {
 
 // particle runs: block b covers the particles of cells [x0, x0 + kx) of one grid row (contiguous
 // in sorted order)
-__device__ __forceinline__ void particle_run(const GridDev& g, int kx, int& h0, int& h1) {
+__device__ __forceinline__ int particle_run(const GridDev& g, int kx, int& h0, int& h1) {
     const int per_row = (g.n[0] + kx - 1) / kx;
     const int row = blockIdx.x / per_row, x0 = (blockIdx.x % per_row) * kx;
     const int base = row * g.n[0];
     h0 = g.off[base + x0];
     h1 = g.off[base + min(x0 + kx, g.n[0])];
+    return base + x0;
 }
 
 }  // namespace pisurf

@@ -46,3 +46,23 @@ def test_merged_samples_equal_single_samples(name, prec, qef):
     assert sa["field_evals"] == sb["field_evals"] and sa["sample_evals"] == sb["sample_evals"]
     if name == "crown":  # more nodes than go by tiles at a point per cell
         assert np.count_nonzero(na["depth"] == ia["depth_min"]) > 1 << 15
+
+
+@pytest.mark.parametrize("prec,qef", [(capi.FP32_KAHAN, 0), (capi.FP64, capi.QEF_REFERENCE)])
+def test_tree_with_the_normals_it_reads(prec, qef):
+    """From 2^20 particles on a tree takes the normals of the cells that its curvatures read; the same tree as
+    with every normal there before."""
+    xyz, r = FRAMES["crown"]()
+    assert len(xyz) >= 1 << 20
+    out = []
+    for before in (False, True):
+        ctx = gpu_context(xyz, r, precision=prec, qef_mode=qef)
+        if before:
+            ctx.particle_normals()
+        info = ctx.build_tree()
+        out.append((info, ctx.tree_nodes(info["n_nodes"]), ctx.stats()["grad_evals"]))
+        ctx.close()
+    (ia, na, ga), (ib, nb, gb) = out
+    assert ia == ib and ga == gb
+    for key in ("type", "id", "depth", "child", "node"):
+        assert np.array_equal(na[key], nb[key]), key
