@@ -977,7 +977,8 @@ int sweep(pisurf_ctx* c, LevelBuf* L, int32_t* sc_dev, int level_depth) {
     if (split_curv)
         launch_empty_curv(c->g, c->spos.as<float4>(), c->nrm.as<float4>(), tp, v, group, kCurvOnly, c->samples.p,
                           (int)rsz, c->stream);
-    launch_classify(prec, c->g, c->rec_a.p, c->rec_g.p, fc, tp, v, c->samples.p, sc_dev, c->ctr(), c->stream);
+    launch_classify(prec, c->g, c->rec_a.p, c->rec_g.p, fc, tp, v, c->samples.p, sc_dev,
+                    level_depth >= 0 ? lattice_density(c, level_depth, 1) : 0.0, c->ctr(), c->stream);
     HIPCHK(c, hipGetLastError());
     return PISURF_OK;
 }
@@ -1059,7 +1060,7 @@ int top_levels_issue(pisurf_ctx* c, hipStream_t s, DBuf& tmp) {
             const int group = (w * w <= 6) ? 4 : (w * w <= 8) ? 8 : (w * w <= 16) ? 16 : 64;
             launch_empty_curv(c->g, c->spos.as<float4>(), c->nrm.as<float4>(), tp, v, group, kEmptyAndCurv, nullptr, 0,
                               s);
-            launch_classify(prec, c->g, c->rec_a.p, c->rec_g.p, fc, tp, v, c->samples.p, nullptr, c->ctr(), s);
+            launch_classify(prec, c->g, c->rec_a.p, c->rec_g.p, fc, tp, v, c->samples.p, nullptr, 0.0, c->ctr(), s);
             exclusive_scan_i32(L->flag.as<int>(), L->scanned.as<int>(), ub[l] + 1, tmp.as<int>(), s);
             launch_children_counted(v, L->scanned.as<int>(), c->levels[l + 1]->view(), cnt + l + 1, s);
         }
@@ -2057,7 +2058,7 @@ int batch_level_classify(BatchFrame& f, BatchReads& br) {
     if (f.split_curv)
         launch_empty_curv(c->g, c->spos.as<float4>(), c->nrm.as<float4>(), f.tp, v, f.group, kCurvOnly, c->samples.p,
                           (int)rsz, c->stream);
-    launch_classify(prec, c->g, c->rec_a.p, c->rec_g.p, field_const(c), f.tp, v, c->samples.p, nullptr, c->ctr(),
+    launch_classify(prec, c->g, c->rec_a.p, c->rec_g.p, field_const(c), f.tp, v, c->samples.p, nullptr, 0.0, c->ctr(),
                     c->stream);
     launch_fill_i32(L->flag.as<int>() + L->n, 1, 0, c->stream);
     exclusive_scan_i32(L->flag.as<int>(), L->scanned.as<int>(), L->n + 1, c->tmp.as<int>(), c->stream);

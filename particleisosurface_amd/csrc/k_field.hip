@@ -16,8 +16,8 @@ template <class R> struct PointSrc {
     double* f;
     double* grad;
     R iso, sigma;
-    __device__ __forceinline__ bool point(int64_t i, float p[3]) const {
-        for (int a = 0; a < 3; a++) p[a] = q[3 * i + a];
+    __device__ __forceinline__ bool point(int64_t i, R p[3]) const {
+        for (int a = 0; a < 3; a++) p[a] = R(q[3 * i + a]);
         return true;
     }
     __device__ __forceinline__ void store(int64_t i, int c, R v) const {

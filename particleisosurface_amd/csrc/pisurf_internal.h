@@ -280,9 +280,10 @@ void launch_samples(int prec, GridDev g, const void* rec_a, const void* rec_g, F
                     NodeLevel lv, const int* list, const int* count, void* samples /*n*27 R*/, Counters* ctr,
                     hipStream_t s);
 // node types, vertices and values, and lv.flag (1 for an internal node; lv.flag[lv.n] = 0 closes
-// the flags for their scan)
+// the flags for their scan); node_density: nodes per hash cell
 void launch_classify(int prec, GridDev g, const void* rec_a, const void* rec_g, FieldConst fc, TreeParams tp,
-                     NodeLevel lv, const void* samples, int32_t* signchange, Counters* ctr, hipStream_t s);
+                     NodeLevel lv, const void* samples, int32_t* signchange, double node_density, Counters* ctr,
+                     hipStream_t s);
 void launch_children(NodeLevel parent, const int* scanned, NodeLevel next, hipStream_t s);
 // the same for a parent level with a device count (parent.ndev, parent.n its upper bound): the
 // children's count 8 * scanned[parent.n] is written to *next_count

@@ -28,8 +28,8 @@ template <class R, bool GRAD> struct PointLds {
     int list[2 * kWave];
 };
 
-// Points i0 .. i0 + np - 1 of src (np <= points_per_wave; i0 and np uniform over the wave): bool point(i, q) gives a
-// point's position or says that there is none, store(i, c, v) takes its sum c (field, then gradient). Returns the
+// Points i0 .. i0 + np - 1 of src (np <= points_per_wave; i0 and np uniform over the wave): bool point(i, p) gives a
+// point's position (R or float) or says that there is none, the same in every lane; store(i, c, v) takes its sum c (field, then gradient). Returns the
 // candidates visited and adds the points evaluated to evals.
 template <class R, bool K, bool GRAD, int MODE, class Src>
 __device__ __forceinline__ unsigned long long point_eval(const GridDev& g, const Recs<R>& rec, const FieldConst& fc,
@@ -53,13 +53,12 @@ __device__ __forceinline__ unsigned long long point_eval(const GridDev& g, const
     };
     unsigned long long vis = 0;
     for (int k = 0; k < np; k++) {
-        float q[3];
-        if (!src.point(i0 + k, q)) continue;
-        const float x = q[0], y = q[1], z = q[2];
+        R p[3];
+        if (!src.point(i0 + k, p)) continue;
         evals++;
-        const R px = R(x), py = R(y), pz = R(z);
+        const R px = p[0], py = p[1], pz = p[2];
         int ix, iy, iz, lo = 0, hi = 0;
-        cell_of(g, x, y, z, ix, iy, iz);
+        cell_of(g, float(px), float(py), float(pz), ix, iy, iz);
         if (lane >= 9 || !row_range(g, ix, iy, iz, lane, lo, hi)) lo = hi = 0;
         int end = hi - lo;
 #pragma unroll

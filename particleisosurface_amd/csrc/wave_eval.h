@@ -126,11 +126,12 @@ __device__ __forceinline__ void wave_cull(const float4* cull, const WavePoints& 
 // Adds to st the contributions of the candidates of point p (act: the lane has a point) and returns
 // their number, passing or not. Every lane of the wave calls it. Neighbouring lanes should lie close
 // together; any order is right unless kWaveSorted is given, which says that the points come in cell order,
-// active lanes first. BACK: cells before the first lane's that its row piece may take.
+// active lanes first. BACK: cells before the first lane's that its row piece may take. p is the position that picks the
+// cell, q the one that distances are taken from (the same, or p before it was rounded to float).
 constexpr int kWaveSorted = -1;
 template <int BACK, class Pol>
 __device__ __forceinline__ int wave_visit(const GridDev& g, const Pol& pol, typename Pol::State& st, bool act,
-                                          const float p[3], WaveLds<Pol>& L) {
+                                          const float p[3], const typename Pol::Real q[3], WaveLds<Pol>& L) {
     typedef typename Pol::Real Real;
     const int lane = threadIdx.x & (kWave - 1);
     int ix, iy, iz;
@@ -209,7 +210,7 @@ __device__ __forceinline__ int wave_visit(const GridDev& g, const Pol& pol, type
         const float ox = g.b0[0] + 0.5f * float(x0 + x1 + 1) * g.cell, oy = g.b0[1] + (float(ly) + 0.5f) * g.cell,
                     oz = g.b0[2] + (float(lz) + 0.5f) * g.cell;
         WavePoints pt;
-        pt.set((p[0] - ox) * ic, (p[1] - oy) * ic, (p[2] - oz) * ic);
+        pt.set(float(q[0] - Real(ox)) * ic, float(q[1] - Real(oy)) * ic, float(q[2] - Real(oz)) * ic);
         for (int cb = 0; cb < total; cb += Pol::kChunk) {
             const int n = min((int)Pol::kChunk, total - cb);
             // batches of 64 nb slots, words of wl
@@ -395,12 +396,26 @@ __device__ __forceinline__ int wave_eval(const GridDev& g, const Recs<R>& rec, c
     const int h = (int)blockIdx.x * T + (int)threadIdx.x;
     float p[3] = {0.f, 0.f, 0.f};
     const bool act = h < n && src.point(h, p);
-    typename WaveField<R, K, GRAD, MODE>::State st{R(p[0]), R(p[1]), R(p[2])};
-    const int ncand = wave_visit<BACK>(g, pol, st, act, p, lds[threadIdx.x / kWave]);
+    const R q[3] = {R(p[0]), R(p[1]), R(p[2])};
+    typename WaveField<R, K, GRAD, MODE>::State st{q[0], q[1], q[2]};
+    const int ncand = wave_visit<BACK>(g, pol, st, act, p, q, lds[threadIdx.x / kWave]);
     if (act) {
         const R gr[3] = {st.ga[0].get(), st.ga[1].get(), st.ga[2].get()};
         src.store(h, st.acc.get(), gr);
     }
+    return ncand;
+}
+
+// The sum at one position q per lane (act: the lane has one); neighbouring lanes should lie close together. Returns the
+// candidates of this lane's point.
+template <class R, bool K, int MODE>
+__device__ __forceinline__ int wave_sum(const GridDev& g, const Recs<R>& rec, const FieldConst& fc, bool act,
+                                        const R q[3], WaveLds<WaveField<R, K, false, MODE>>& lds, R& sum) {
+    const WaveField<R, K, false, MODE> pol(rec, fc);
+    const float p[3] = {float(q[0]), float(q[1]), float(q[2])};
+    typename WaveField<R, K, false, MODE>::State st{q[0], q[1], q[2]};
+    const int ncand = wave_visit<kWaveCells / 2>(g, pol, st, act, p, q, lds);
+    sum = st.acc.get();
     return ncand;
 }
 

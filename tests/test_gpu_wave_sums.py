@@ -107,3 +107,39 @@ def test_points_match_oracle(prec):
     assert np.max(np.abs(f - f2)) <= tol * np.max(np.abs(iso - f2) + iso)
     assert np.max(np.abs(g - g2)) <= tol * np.max(np.abs(g2))
     ctx.close()
+
+
+@pytest.mark.parametrize("prec", [capi.FP32_KAHAN, capi.FP64])
+def test_many_edges_equal_few_edges(frame, prec):
+    """2^16 edges or more take a thread each, fewer a wave per one to eight edges: the same vertices and counts."""
+    xyz, r = frame
+    s = synth.Stream(29)
+    n = (1 << 16) + 5
+    pick = (s.uniform(n) * len(xyz)).astype(np.int64)
+    a = (xyz[pick] + s.uniform(3 * n, -2 * r, 2 * r).reshape(-1, 3)).astype(np.float32)
+    b = a + np.float32(2 * r) * np.eye(3, dtype=np.float32)[np.arange(n) % 3]
+    ctx = gpu_context(xyz, r, precision=prec)
+    ends = np.stack([np.concatenate([p, ctx.eval_points(p)[:, None]], axis=1) for p in (a, b)], axis=1)
+    ends[3] = ends[3, 0]  # no length: no step
+    whole = ctx.bisect_edges(ends)
+    for lo, hi in ((0, 3), (1000, 6000), (0, (1 << 16) - 1)):
+        part = ctx.bisect_edges(ends[lo:hi])
+        assert np.array_equal(whole[0][lo:hi], part[0], equal_nan=True) and np.array_equal(whole[1][lo:hi], part[1])
+    ctx.close()
+
+
+@pytest.mark.parametrize("ani,poly6", [(True, False), (False, True)])
+@pytest.mark.parametrize("scene", ["sphere", "dam"])
+def test_qef_vertex_values_equal_point_values(scene, ani, poly6):
+    """Vertex values of leaves, by waves of nodes in the deepest levels and point by point above them."""
+    xyz, r = synth.lattice_sphere(radius=0.05, r=0.005) if scene == "sphere" else synth.dam_break()
+    ctx = gpu_context(xyz, r, use_ani=ani, use_poly6=poly6, qef_mode=capi.QEF_REFERENCE)
+    info = ctx.run_frame()
+    nodes = ctx.tree_nodes(info["n_nodes"])
+    pick = (nodes["type"] == 2) & (nodes["depth"] >= info["depth_min"])
+    v = nodes["node"][pick]
+    f = ctx.eval_points(v[:, :3].astype(np.float32))
+    ctx.close()
+    assert len(v) > 1000
+    assert np.array_equal(v[:, :3], v[:, :3].astype(np.float32).astype(np.float64))
+    assert np.all((v[:, 3] == f) | (v[:, 3] == 0)) and np.count_nonzero(v[:, 3]) > len(v) // 4
