@@ -6,6 +6,7 @@
 #include "run_tuner.h"
 #include "wave_eval.h"
 
+#include <cmath>
 #include <type_traits>
 
 namespace pisurf {
@@ -251,6 +252,20 @@ void launch_normals(int prec, GridDev g, const void* ra, const void* rg, FieldCo
 // UniformGrid::gridSampling (src/marching.cpp:72-91): point i = x + dims0 * (y + dims1 * z) at
 // float(steps - x) / float(steps) * min + float(x) / float(steps) * max per axis, each operation
 // rounded on its own (the reference is built without FMA contraction)
+__device__ __forceinline__ void lattice_point(const UniformBox& ub, const int ix[3], float p[3]) {
+#pragma unroll
+    for (int a = 0; a < 3; a++) {
+        // plain operators with contraction off in this scope: the *_rn helpers are inlined as
+        // contractable operations, and a fused product would round differently
+#pragma clang fp contract(off)
+        const float st = (float)ub.steps[a];
+        const float u = (float)(ub.steps[a] - ix[a]) / st;
+        const float v = (float)ix[a] / st;
+        p[a] = u * ub.lo[a] + v * ub.hi[a];
+    }
+}
+
+// One thread per point, for hash cells too small to hold several
 template <class R, bool K>
 __global__ void __launch_bounds__(256) k_uniform_grid(GridDev g, Recs<R> rec, FieldConst fc, UniformBox ub,
                                                       int64_t total, float* __restrict__ out, Counters* ctr) {
@@ -261,19 +276,9 @@ __global__ void __launch_bounds__(256) k_uniform_grid(GridDev g, Recs<R> rec, Fi
         const int z = (int)(i / plane);
         const int64_t rem = i - (int64_t)z * plane;
         const int y = (int)(rem / ub.dims[0]);
-        const int x = (int)(rem - (int64_t)y * ub.dims[0]);
-        const int ix[3] = {x, y, z};
+        const int ix[3] = {(int)(rem - (int64_t)y * ub.dims[0]), y, z};
         float p[3];
-#pragma unroll
-        for (int a = 0; a < 3; a++) {
-            // plain operators with contraction off in this scope: the *_rn helpers are inlined as
-            // contractable operations, and a fused product would round differently
-#pragma clang fp contract(off)
-            const float st = (float)ub.steps[a];
-            const float u = (float)(ub.steps[a] - ix[a]) / st;
-            const float v = (float)ix[a] / st;
-            p[a] = u * ub.lo[a] + v * ub.hi[a];
-        }
+        lattice_point(ub, ix, p);
         R s, gr[3];
         vis = field_sum<R, K, false>(g, rec, fc, p[0], p[1], p[2], R(p[0]), R(p[1]), R(p[2]), s, gr);
         out[i] = float(field_value(R(fc.iso), out_sigma<R, K>(fc), s));
@@ -282,18 +287,72 @@ __global__ void __launch_bounds__(256) k_uniform_grid(GridDev g, Recs<R> rec, Fi
     wave_count(&ctr_stripe(ctr)->candidates, (unsigned long long)vis);
 }
 
+// A wave per block of 4 x 4 x 4 points. The lattice has four points to a hash cell's width (spacing r, cells of 4 r), and
+// the blocks start where cells do (shift), so a wave's points nearly always share one window: 216 candidates staged
+// and tested once for 64 points (wave_eval.h). Four blocks side by side along x per workgroup.
+// 2 M points around 120 k particles, FP32: 260 us, a thread per point 426.
+struct LatticeBlocks {
+    int shift[3];  // points of the first block along an axis that lie before the lattice
+    int n[3];      // blocks (x: groups of four)
+};
+template <class R, bool K, int MODE>
+__global__ void __launch_bounds__(256) k_wave_lattice(GridDev g, Recs<R> rec, FieldConst fc, UniformBox ub,
+                                                      LatticeBlocks lb, float* __restrict__ out, Counters* ctr) {
+    __shared__ WaveLds<WaveField<R, K, false, MODE>> lds[4];
+    const int lane = threadIdx.x & (kWave - 1), w = threadIdx.x / kWave;
+    const int b = blockIdx.x, bx = b % lb.n[0], by = (b / lb.n[0]) % lb.n[1], bz = b / lb.n[0] / lb.n[1];
+    const int ix[3] = {16 * bx + 4 * w + (lane & 3) - lb.shift[0], 4 * by + ((lane >> 2) & 3) - lb.shift[1],
+                       4 * bz + (lane >> 4) - lb.shift[2]};
+    bool act = true;
+#pragma unroll
+    for (int a = 0; a < 3; a++) act = act && ix[a] >= 0 && ix[a] < ub.dims[a];
+    float p[3] = {0.f, 0.f, 0.f};
+    if (act) lattice_point(ub, ix, p);
+    const R q[3] = {R(p[0]), R(p[1]), R(p[2])};
+    R sum;
+    const int vis = wave_sum<R, K, MODE>(g, rec, fc, act, q, lds[w], sum);
+    if (act)
+        out[((int64_t)ix[2] * ub.dims[1] + ix[1]) * ub.dims[0] + ix[0]] =
+            float(field_value(R(fc.iso), out_sigma<R, K>(fc), sum));
+    wave_count(&ctr_stripe(ctr)->field_evals, act ? 1ull : 0ull);
+    wave_count(&ctr_stripe(ctr)->candidates, (unsigned long long)vis);
+}
+
 void launch_uniform_grid(int prec, GridDev g, const void* ra, const void* rg, FieldConst fc, UniformBox ub,
                          int64_t total, float* out, Counters* ctr, hipStream_t s) {
     if (total <= 0) return;
-    const unsigned nb = (unsigned)((total + 255) / 256);
-    if (prec == 2) {
-        Recs<double> r{(const double4*)ra, (const double4*)rg};
-        k_uniform_grid<double, false><<<nb, 256, 0, s>>>(g, r, fc, ub, total, out, ctr);
-    } else {
-        Recs<float> r{(const float4*)ra, (const float4*)rg};
-        if (prec == 1) k_uniform_grid<float, true><<<nb, 256, 0, s>>>(g, r, fc, ub, total, out, ctr);
-        else k_uniform_grid<float, false><<<nb, 256, 0, s>>>(g, r, fc, ub, total, out, ctr);
+    LatticeBlocks lb;
+    double per_cell = 1;
+    int64_t blocks = 1;
+    for (int a = 0; a < 3; a++) {
+        const double h = ((double)ub.hi[a] - ub.lo[a]) / ub.steps[a];
+        per_cell *= g.cell / h;
+        const double at = ((double)g.b0[a] - ub.lo[a]) / h;  // lattice position of a cell's first point, modulo 4
+        const double first = std::ceil(at - 4 * std::floor(at / 4) - 1e-3);
+        lb.shift[a] = std::isfinite(first) ? (4 - (int)first) & 3 : 0;
+        const int width = a == 0 ? 16 : 4;
+        lb.n[a] = (ub.dims[a] + lb.shift[a] + width - 1) / width;
+        blocks *= lb.n[a];
     }
+    // (cells of another size: 64 points in more than 16 cells share too little)
+    const bool waves = per_cell >= kWaveDensity && blocks <= INT32_MAX;
+    const unsigned nb = (unsigned)((total + 255) / 256);
+    auto go = [&](auto mode) {
+        constexpr int M = decltype(mode)::value;
+        if (prec == 2) {
+            Recs<double> r{(const double4*)ra, (const double4*)rg};
+            if (waves) k_wave_lattice<double, false, M><<<(unsigned)blocks, 256, 0, s>>>(g, r, fc, ub, lb, out, ctr);
+            else k_uniform_grid<double, false><<<nb, 256, 0, s>>>(g, r, fc, ub, total, out, ctr);
+        } else {
+            Recs<float> r{(const float4*)ra, (const float4*)rg};
+            if (prec == 1 && waves)
+                k_wave_lattice<float, true, M><<<(unsigned)blocks, 256, 0, s>>>(g, r, fc, ub, lb, out, ctr);
+            else if (prec == 1) k_uniform_grid<float, true><<<nb, 256, 0, s>>>(g, r, fc, ub, total, out, ctr);
+            else if (waves) k_wave_lattice<float, false, M><<<(unsigned)blocks, 256, 0, s>>>(g, r, fc, ub, lb, out, ctr);
+            else k_uniform_grid<float, false><<<nb, 256, 0, s>>>(g, r, fc, ub, total, out, ctr);
+        }
+    };
+    point_dispatch(field_mode(fc), go);
 }
 
 }  // namespace pisurf

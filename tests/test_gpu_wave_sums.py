@@ -143,3 +143,25 @@ def test_qef_vertex_values_equal_point_values(scene, ani, poly6):
     assert len(v) > 1000
     assert np.array_equal(v[:, :3], v[:, :3].astype(np.float32).astype(np.float64))
     assert np.all((v[:, 3] == f) | (v[:, 3] == 0)) and np.count_nonzero(v[:, 3]) > len(v) // 4
+
+
+@pytest.mark.parametrize("prec", [capi.FP32, capi.FP32_KAHAN, capi.FP64])
+@pytest.mark.parametrize("inf_factor", [4.0, 5.3, 1.0])
+def test_lattice_equals_point_values(prec, inf_factor):
+    """The dense lattice by waves of 4 x 4 x 4 points (cells of 4 r: one window per wave, of 5.3 r: blocks across
+    cells) and a thread per point (cells of r), against the field at the same points."""
+    xyz, r = synth.random_cloud(1500, r=0.01, extent=0.23)
+    ctx = gpu_context(xyz, r, precision=prec)
+    if inf_factor != 4.0:
+        ctx.hashgrid_build(inf_factor=inf_factor)
+    vals, box, sp = ctx.uniform_grid()
+    nz, ny, nx = vals.shape
+    f32 = np.float32
+    axes = []
+    for a, n in enumerate((nx, ny, nz)):
+        i, st = np.arange(n), f32(n - 1)
+        axes.append((f32(n - 1 - i) / st) * f32(box[2 * a]) + (i.astype(f32) / st) * f32(box[2 * a + 1]))
+    z, y, x = np.meshgrid(axes[2], axes[1], axes[0], indexing="ij")
+    f = ctx.eval_points(np.stack([x, y, z], axis=-1).astype(f32).reshape(-1, 3))
+    ctx.close()
+    assert np.array_equal(vals.reshape(-1), f.astype(f32))
