@@ -331,10 +331,10 @@ def main():
                                             st["ms_normals"] / args.steps, st["ms_tree"] / args.steps,
                                             st["ms_extract_host"] / args.steps, st["ms_bisect"] / args.steps))
     performed = st["sample_unique"] if st["sample_unique"] > 0 else st["sample_evals"]
-    performed_per_frame = (evals_per_frame - st["sample_evals"] + performed) // args.steps
+    performed_per_frame = (evals_per_frame - st["grad_evals"] - st["sample_evals"] + performed) // args.steps
     # the headline: field evaluations the device performed per second of frame time (node samples
-    # shared by neighbouring nodes are evaluated once); the reference's count (27 per sampled node)
-    # is reported beside it
+    # shared by the nodes of a tile are evaluated once; normals are left out, as a tree takes only those
+    # that it reads); the reference's count (27 per sampled node, every normal) is reported beside it
     value = performed_per_frame / (dt / args.steps)
 
     # roofline of the dominant field-evaluation kernel, the node-sampling kernel. Its limiter is VALU
@@ -368,7 +368,8 @@ def main():
                     algorithmic_GBps=round(alg / max(launches, 1) / k_s / 1e9, 1) if k_s > 0 else None)
         return roof
     if st["run_launches"] > 0:
-        roof = kernel_roof("k_run_samples", st["run_evals"], st["run_candidates"], st["run_launches"],
+        # (the sampling launches: waves, and runs at D_min)
+        roof = kernel_roof("k_wave_samples", st["run_evals"], st["run_candidates"], st["run_launches"],
                            st["ms_run_kernel"])
     else:
         roof = kernel_roof("k_samples", st["sample_evals"], st["sample_candidates"], st["sample_launches"],
