@@ -18,7 +18,8 @@
 //    and wave gathers the sign bits;
 //  - each lane walks its own pass bits over the whole chunk, so a wave takes as many steps as its busiest point has
 //    passing candidates in the chunk (52 at the crown splash's deepest level; word by word it is 70).
-// Deepest level of the crown splash (11.9 M points): 1.20 ms, 60 vector instructions per point, against 1.5 ms and 90.
+// Deepest level of the crown splash (11.9 M points sorted over the level): 1.20 ms, 60 vector instructions per point,
+// against 1.5 ms and 90.
 // A chunk of 224 candidates takes a tenth fewer instructions, but its LDS leaves two waves per SIMD instead of
 // four, and the kernel 1.5 times as long. Sorting the points by their passing candidates before dealing them to
 // the lanes saves a tenth of the instructions (two points per lane) and loses as much to the occupancy.
