@@ -675,6 +675,7 @@ int normals_launch(pisurf_ctx* c) {
                    c->ginfo.n_invalid, nullptr, c->nrm.as<float4>(), c->ctr(), c->trial_ctr(), c->stream);
     HIPCHK(c, hipGetLastError());
     c->normals_done = true;
+    c->normals_at_dmin = false;
     return PISURF_OK;
 }
 
@@ -782,6 +783,9 @@ int tree_ready(pisurf_ctx* c) {
     int rc = need_aniso(c);
     if (rc) return rc;
     if (!c->consts_done) compute_constants(c);
+    // (a depth override of 1 or 2 puts D_min above the root: every level reads curvatures, none is D_min)
+    resize_root(c);
+    if (c->dmin < 0) return frame_ready(c);
     HIPCHK(c, c->nrm.ensure(c->n * sizeof(float4)));
     c->normals_at_dmin = true;
     return PISURF_OK;
@@ -826,6 +830,8 @@ int sweep(pisurf_ctx* c, LevelBuf* L, int32_t* sc_dev, int level_depth) {
     // samples change sign; deeper levels hold the children of such nodes, and mixed API sweeps,
     // do both at once. (Above D_min classification reads no curvature.)
     const bool split_curv = level_depth >= 0 && level_depth == c->dmin;
+    if (c->normals_at_dmin && tp.curv && tp.calc_normals && !split_curv && (level_depth < 0 || level_depth > c->dmin))
+        return c->fail(PISURF_E_STATE, "curvature without the normals it reads");
     launch_empty_curv(c->g, c->spos.as<float4>(), c->nrm.as<float4>(), tp, v, group,
                       split_curv ? kEmptyOnly : kEmptyAndCurv, nullptr, 0, c->stream);
     // the level's flag / scanned / child arrays serve as the sample list until classification
