@@ -251,7 +251,8 @@ struct pisurf_ctx {
     // normals
     bool normals_done = false;
     bool normals_at_dmin = false;  // the tree takes the normals it reads when D_min is sampled
-    DBuf cmark;                    // a byte per cell: its normals are needed
+    bool normals_some = false;     // the normals of the cells marked in cmark are there
+    DBuf cmark;                    // a byte per cell: 1 its normals are needed, 2 they are there
     DBuf nrm;
     // tree
     bool tree_done = false;
@@ -617,7 +618,7 @@ void aniso_finish(pisurf_ctx* c, unsigned long long nfp) {
     c->n_fp64_eig = nfp;
     c->prec_rec = prec_of(c);
     c->aniso_done = true;
-    c->normals_done = c->tree_done = false;
+    c->normals_done = c->normals_some = c->tree_done = false;
 }
 
 int do_aniso(pisurf_ctx* c) {
@@ -672,32 +673,56 @@ int need_aniso(pisurf_ctx* c) {
 int normals_launch(pisurf_ctx* c) {
     HIPCHK(c, c->nrm.ensure(c->n * sizeof(float4)));
     launch_normals(prec_of(c), c->g, c->rec_a.p, c->rec_g.p, field_const(c), c->spos.as<float4>(), c->n,
-                   c->ginfo.n_invalid, nullptr, c->nrm.as<float4>(), c->ctr(), c->trial_ctr(), c->stream);
+                   c->ginfo.n_invalid, nullptr, true, c->nrm.as<float4>(), c->ctr(), c->trial_ctr(), c->stream);
     HIPCHK(c, hipGetLastError());
     c->normals_done = true;
     c->normals_at_dmin = false;
     return PISURF_OK;
 }
 
+int64_t mark_words(const pisurf_ctx* c) { return ((int64_t)c->g.n[0] * c->g.n[1] * c->g.n[2] + 3) / 4; }
+
+// The normals of the runs with a cell marked 1, and the cells marked as there. The first such launch counts every
+// particle's, as the reference takes them all once, and later ones none.
+int marked_normals_launch(pisurf_ctx* c) {
+    launch_normals(prec_of(c), c->g, c->rec_a.p, c->rec_g.p, field_const(c), c->spos.as<float4>(), c->n,
+                   c->ginfo.n_invalid, c->cmark.as<uint8_t>(), !c->normals_some, c->nrm.as<float4>(), c->ctr(),
+                   c->trial_ctr(), c->stream);
+    launch_marks_taken(c->cmark.as<uint32_t>(), mark_words(c), c->stream);
+    HIPCHK(c, hipGetLastError());
+    c->normals_some = true;
+    c->normals_at_dmin = false;
+    return PISURF_OK;
+}
+
+// the normals that trees have not taken
+int normals_rest(pisurf_ctx* c) {
+    const double t0 = now_ms();
+    launch_marks_rest(c->cmark.as<uint32_t>(), mark_words(c), c->stream);
+    const int rc = marked_normals_launch(c);
+    if (rc) return rc;
+    c->normals_done = true;
+    HIPCHK(c, c->wait());
+    c->st.ms_normals += now_ms() - t0;
+    return PISURF_OK;
+}
+
 // The normals that the curvatures of a tree can read, once D_min's samples are there: curvature is taken for the
 // sampled D_min nodes whose samples change sign and for their descendants (the others are leaves), and sums
 // normals over a node's grown box. A fluid's inside needs none: frames of 1.1 M, 4 M (crown splashes) and 12 M
-// particles take 0.06, 0.13 and 1.06 ms less.
+// particles take 0.06, 0.13 and 1.06 ms less. They stay with the particles: another tree on them takes only the
+// cells that no tree before it read (4 M particles, the same tree again: 6.03 -> 5.57 ms).
 int normals_for_tree(pisurf_ctx* c, const TreeParams& tp, const NodeLevel& lv, int rsz) {
-    const int64_t ncell = (int64_t)c->g.n[0] * c->g.n[1] * c->g.n[2];
-    HIPCHK(c, c->cmark.ensure((ncell + 3) / 4 * 4));
-    launch_fill_i32(c->cmark.as<int>(), (ncell + 3) / 4, 0, c->stream);
+    if (!c->normals_some) {
+        HIPCHK(c, c->cmark.ensure(mark_words(c) * 4));
+        launch_fill_i32(c->cmark.as<int>(), mark_words(c), 0, c->stream);
+    }
     float most = 0;
     for (int a = 0; a < 3; a++)
         most = std::max({most, std::fabs(c->root_c[a]) + c->root_half, std::fabs(c->g.b0[a])});
     launch_mark_cells(c->g, tp, lv, c->samples.p, rsz, 0.01f * c->g.cell + 4e-6f * most, c->cmark.as<uint8_t>(),
                       c->stream);
-    launch_normals(prec_of(c), c->g, c->rec_a.p, c->rec_g.p, field_const(c), c->spos.as<float4>(), c->n,
-                   c->ginfo.n_invalid, c->cmark.as<uint8_t>(), c->nrm.as<float4>(), c->ctr(), c->trial_ctr(),
-                   c->stream);
-    HIPCHK(c, hipGetLastError());
-    c->normals_at_dmin = false;
-    return PISURF_OK;
+    return marked_normals_launch(c);
 }
 
 int top_levels_read(pisurf_ctx* c);
@@ -764,12 +789,13 @@ int frame_ready(pisurf_ctx* c) {
     if (rc) return rc;
     if (!c->consts_done) compute_constants(c);
     if (c->prm.calc_normals && !c->normals_done) {
-        rc = do_normals(c);
+        rc = c->normals_some ? normals_rest(c) : do_normals(c);
         if (rc) return rc;
     }
     if (!c->normals_done) {  // curvature reads normals; without CALC_P_NORMAL they stay zero
         HIPCHK(c, c->nrm.ensure(c->n * sizeof(float4)));
         HIPCHK(c, hipMemsetAsync(c->nrm.p, 0, c->n * sizeof(float4), c->stream));
+        c->normals_some = false;
     }
     return PISURF_OK;
 }
@@ -779,9 +805,11 @@ int frame_ready(pisurf_ctx* c) {
 constexpr int64_t kTreeNormalsMin = int64_t(1) << 20;
 int tree_ready(pisurf_ctx* c) {
     c->normals_at_dmin = false;
-    if (!c->prm.calc_normals || c->normals_done || c->n < kTreeNormalsMin) return frame_ready(c);
+    if (!c->prm.calc_normals || c->n < kTreeNormalsMin) return frame_ready(c);
     int rc = need_aniso(c);
     if (rc) return rc;
+    // (with particles outside the grid all are taken, one thread each)
+    if (c->normals_done || c->ginfo.n_invalid > 0) return frame_ready(c);
     if (!c->consts_done) compute_constants(c);
     // (a depth override of 1 or 2 puts D_min above the root: every level reads curvatures, none is D_min)
     resize_root(c);

@@ -81,18 +81,18 @@ template <class R> struct ParticleSrc {
 template <class R, bool K, int T, int MODE>
 __global__ void __launch_bounds__(T) k_run_normals(GridDev g, Recs<R> rec, FieldConst fc,
                                                    const float4* __restrict__ spos, int kx,
-                                                   const uint8_t* __restrict__ mark, float4* __restrict__ nrm,
-                                                   Counters* ctr) {
+                                                   const uint8_t* __restrict__ mark, bool count,
+                                                   float4* __restrict__ nrm, Counters* ctr) {
     __shared__ RunLds<R, K && sizeof(R) == 4> lds;
     int h0, h1;
     const int cell = particle_run(g, kx, h0, h1);
     if (h0 >= h1) return;  // uniform over the block
     // (the count is the reference's, which takes every particle's normal)
-    if (threadIdx.x == 0) atomicAdd(&ctr_stripe(ctr)->grad_evals, (unsigned long long)(h1 - h0));
+    if (count && threadIdx.x == 0) atomicAdd(&ctr_stripe(ctr)->grad_evals, (unsigned long long)(h1 - h0));
     if (mark) {
         const int nc = min(kx, g.n[0] - cell % g.n[0]);
         bool any = false;
-        for (int x = threadIdx.x; x < nc; x += T) any = any || mark[cell + x];
+        for (int x = threadIdx.x; x < nc; x += T) any = any || mark[cell + x] == 1;
         if (!__syncthreads_or(any)) return;
     }
     ParticleSrc<R> src{spos, nrm, out_sigma<R, K>(fc)};
@@ -206,8 +206,8 @@ void launch_eval_points_sorted(int prec, GridDev g, const void* ra, const void* 
 }
 
 void launch_normals(int prec, GridDev g, const void* ra, const void* rg, FieldConst fc, const float4* spos, int64_t n,
-                    int64_t n_invalid, const uint8_t* mark, float4* nrm, Counters* ctr, Counters* trial_ctr,
-                    hipStream_t s) {
+                    int64_t n_invalid, const uint8_t* mark, bool count, float4* nrm, Counters* ctr,
+                    Counters* trial_ctr, hipStream_t s) {
     if (n <= 0) return;
     if (n_invalid > 0) {
         const unsigned nb = (unsigned)((n + 255) / 256);
@@ -234,11 +234,11 @@ void launch_normals(int prec, GridDev g, const void* ra, const void* rg, FieldCo
                 constexpr int TT = decltype(tag)::value, M = decltype(mode)::value;
                 if (prec == 2) {
                     Recs<double> r{(const double4*)ra, (const double4*)rg};
-                    k_run_normals<double, false, TT, M><<<nb, TT, 0, s>>>(g, r, fc, spos, c.kx, mark, nrm, cc);
+                    k_run_normals<double, false, TT, M><<<nb, TT, 0, s>>>(g, r, fc, spos, c.kx, mark, count, nrm, cc);
                 } else {
                     Recs<float> r{(const float4*)ra, (const float4*)rg};
-                    if (prec == 1) k_run_normals<float, true, TT, M><<<nb, TT, 0, s>>>(g, r, fc, spos, c.kx, mark, nrm, cc);
-                    else k_run_normals<float, false, TT, M><<<nb, TT, 0, s>>>(g, r, fc, spos, c.kx, mark, nrm, cc);
+                    if (prec == 1) k_run_normals<float, true, TT, M><<<nb, TT, 0, s>>>(g, r, fc, spos, c.kx, mark, count, nrm, cc);
+                    else k_run_normals<float, false, TT, M><<<nb, TT, 0, s>>>(g, r, fc, spos, c.kx, mark, count, nrm, cc);
                 }
             };
             using M0 = std::integral_constant<int, kModeAny>;

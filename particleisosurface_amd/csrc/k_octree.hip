@@ -177,9 +177,10 @@ __global__ void __launch_bounds__(256) k_empty_curv(GridDev g, const float4* __r
 }
 
 
-// mark[cell] = 1 for the cells whose particles' normals a curvature below this level can read: those of the grown
-// boxes (k_empty_curv) of the sampled nodes whose samples change sign, which hold the grown boxes of all
-// their descendants; slack covers the rounding of the descendants' coordinates. A group of 16 lanes per node.
+// mark[cell] = 1, unless it is 2 (the normals are there), for the cells whose particles' normals a curvature below this
+// level can read: those of the grown boxes (k_empty_curv) of the sampled nodes whose samples change sign, which hold
+// the grown boxes of all their descendants; slack covers the rounding of the descendants' coordinates. A group of 16
+// lanes per node.
 __global__ void __launch_bounds__(256) k_mark_cells(GridDev g, TreeParams tp, NodeLevel lv,
                                                     const void* __restrict__ samples, int rsz, float slack,
                                                     uint8_t* __restrict__ mark) {
@@ -199,8 +200,17 @@ __global__ void __launch_bounds__(256) k_mark_cells(GridDev g, TreeParams tp, No
     if (ny <= 0 || nz <= 0) return;
     for (int row = lane; row < ny * nz; row += 16) {
         const int64_t base = ((int64_t)(lo[2] + row / ny) * g.n[1] + lo[1] + row % ny) * g.n[0];
-        for (int x = lo[0]; x <= hi[0]; x++) mark[base + x] = 1;
+        for (int x = lo[0]; x <= hi[0]; x++)
+            if (mark[base + x] == 0) mark[base + x] = 1;
     }
+}
+
+// four marks a thread: 1 -> 2, or 0 -> 1
+template <bool TAKEN> __global__ void k_marks(uint32_t* __restrict__ mark, int64_t words) {
+    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= words) return;
+    const uint32_t w = mark[i], ones = 0x01010101u;
+    mark[i] = TAKEN ? w + (w & ones) : w | (~(w | (w >> 1)) & ones);
 }
 
 // compaction of the nodes to evaluate: flag, then (after a scan) the list. A listed node gets its
@@ -1281,6 +1291,12 @@ void launch_mark_cells(GridDev g, TreeParams tp, NodeLevel lv, const void* sampl
                        hipStream_t s) {
     if (lv.n <= 0) return;
     k_mark_cells<<<(unsigned)((lv.n + 15) / 16), 256, 0, s>>>(g, tp, lv, samples, rsz, slack, mark);
+}
+void launch_marks_taken(uint32_t* mark, int64_t words, hipStream_t s) {
+    if (words > 0) k_marks<true><<<(unsigned)((words + 255) / 256), 256, 0, s>>>(mark, words);
+}
+void launch_marks_rest(uint32_t* mark, int64_t words, hipStream_t s) {
+    if (words > 0) k_marks<false><<<(unsigned)((words + 255) / 256), 256, 0, s>>>(mark, words);
 }
 
 void launch_sample_list(TreeParams tp, NodeLevel lv, int* flag, int* pos, int* list, int* cflag, int* cpos,

@@ -136,10 +136,11 @@ bool eval_points_sorts(int64_t n, int64_t particles);
 void launch_eval_points_sorted(int prec, GridDev g, const void* rec_a, const void* rec_g, FieldConst fc, const float* q,
                                int64_t n, double* f, double* grad, uint64_t* key, int* val, uint64_t* key2, int* val2,
                                int* tmp, Counters* ctr, hipStream_t s);
-// mark (may be NULL): only the runs with a marked cell. trial_ctr: counter block for the timed trial launches of shape
-// tuning (their counts are not kept)
+// mark (may be NULL): only the runs with a cell marked 1. count: add every particle to the counter. trial_ctr: counter
+// block for the timed trial launches of shape tuning (their counts are not kept)
 void launch_normals(int prec, GridDev g, const void* rec_a, const void* rec_g, FieldConst fc, const float4* spos,
-                    int64_t n, int64_t n_invalid, const uint8_t* mark, float4* nrm, Counters* ctr, Counters* trial_ctr, hipStream_t s);
+                    int64_t n, int64_t n_invalid, const uint8_t* mark, bool count, float4* nrm, Counters* ctr,
+                    Counters* trial_ctr, hipStream_t s);
 // dense sampling box: lo / hi corners, steps (intervals) and dims = steps + 1 points per axis
 struct UniformBox {
     float lo[3], hi[3];
@@ -189,8 +190,11 @@ void launch_empty_curv(GridDev g, const float4* spos, const float4* nrm, TreePar
 void launch_sample_list(TreeParams tp, NodeLevel lv, int* flag, int* pos, int* list, int* cflag, int* cpos,
                         int* clist, int* zero, int* tmp, hipStream_t s, ScanPub pub = ScanPub(),
                         ScanPub cpub = ScanPub());
+// cell marks, a byte each (0, 1 or 2): 1 for the cells below a level's nodes unless 2; every 1 -> 2; every 0 -> 1
 void launch_mark_cells(GridDev g, TreeParams tp, NodeLevel lv, const void* samples, int rsz, float slack, uint8_t* mark,
                        hipStream_t s);
+void launch_marks_taken(uint32_t* mark, int64_t words, hipStream_t s);
+void launch_marks_rest(uint32_t* mark, int64_t words, hipStream_t s);
 void launch_centers(int prec, GridDev g, const void* rec_a, const void* rec_g, FieldConst fc, NodeLevel lv,
                     const int* list, const int* count, void* samples, Counters* ctr, hipStream_t s);
 // the same for k listed centres (count known on the host), grouped by hash cell and evaluated in

@@ -51,3 +51,48 @@ def test_shallow_tree_takes_its_normals(depth):
     assert out[0][0]["depth_max"] == depth and out[0][0]["depth_min"] == depth - 3
     assert_same(*out)
     assert out[0][0]["n_nodes"] == 1
+
+
+@pytest.mark.parametrize("prec", [capi.FP32, capi.FP32_KAHAN, capi.FP64])
+def test_later_trees_keep_the_normals(prec):
+    """Trees built again on the same particles, each reading cells that the ones before did not, then a sweep that reads
+    any: every tree as with all normals there before, every particle's normal counted once."""
+    xyz, r = synth.crown_splash(pool_layers=6, n_drops=20000)
+    assert len(xyz) >= 1 << 20
+    kinds = [dict(smooth_factor=0.5), dict(qef_mode=capi.QEF_REFERENCE), dict(smooth_factor=3.0), dict()]
+    out = []
+    for before in (False, True):
+        ctx = stale_context(xyz, r, precision=prec)
+        if before:
+            ctx.particle_normals()
+        trees = []
+        for kw in kinds:
+            ctx.set_params(r, precision=prec, **kw)
+            trees.append(tree(ctx))
+            assert ctx.stats()["grad_evals"] == len(xyz)
+        nodes = trees[-1][1]
+        pick = np.arange(0, len(nodes["half"]), 97)
+        level = ctx.sweep_level(nodes["center"][pick], nodes["half"][pick], np.full(len(pick), 20))
+        assert ctx.stats()["grad_evals"] == len(xyz)
+        out.append((trees, level))
+        ctx.close()
+    (ta, la), (tb, lb) = out
+    for a, b in zip(ta, tb):
+        assert_same(a, b)
+    for a, b in zip(la, lb):
+        assert np.array_equal(a, b)
+    # the trees differ, so that later ones read more
+    assert len({t[0]["n_nodes"] for t in ta}) > 1
+
+
+def test_normals_left_out_between_trees():
+    """A tree without normals in between clears them: the next tree takes its own again."""
+    xyz, r = synth.crown_splash(pool_layers=6, n_drops=20000)
+    ctx = stale_context(xyz, r)
+    first = tree(ctx)
+    ctx.set_params(r, calc_normals=False)
+    flat = tree(ctx)
+    ctx.set_params(r)
+    assert_same(first, tree(ctx))
+    assert flat[0]["n_nodes"] != first[0]["n_nodes"]
+    ctx.close()
