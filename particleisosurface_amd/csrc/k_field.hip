@@ -225,7 +225,7 @@ void launch_normals(int prec, GridDev g, const void* ra, const void* rg, FieldCo
     // tuned per precision and average particles per cell
     const double p = (double)n / std::max<int64_t>((int64_t)g.n[0] * g.n[1] * g.n[2], 1);
     tuned_run_launch(
-        prec, kRunNormals, p, false, trial_ctr, s,
+        prec, mark ? kRunMarkedNormals : kRunNormals, p, false, trial_ctr, s,
         [&](RunShape c) { return (int64_t)((g.n[0] + c.kx - 1) / c.kx) * g.n[1] * g.n[2] <= INT32_MAX; },
         [&](RunShape c, bool trial) {
             Counters* cc = trial ? trial_ctr : ctr;

@@ -73,7 +73,9 @@ inline std::vector<RunShape> run_shape_candidates(double p, bool wave) {
     return c;
 }
 
-enum RunKind { kRunSamples = 0, kRunCenters = 1, kRunNormals = 2 };
+// kRunMarkedNormals: the runs with a marked cell only, most others empty of work; a shape that suits them says nothing
+// about all particles' normals. (4 and more: the kinds by waves)
+enum RunKind { kRunSamples = 0, kRunCenters = 1, kRunNormals = 2, kRunMarkedNormals = 3 };
 
 class RunTuner {
   public:

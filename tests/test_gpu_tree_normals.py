@@ -96,3 +96,18 @@ def test_normals_left_out_between_trees():
     assert_same(first, tree(ctx))
     assert flat[0]["n_nodes"] != first[0]["n_nodes"]
     ctx.close()
+
+
+def test_a_tree_and_all_normals_tune_apart():
+    """The shape kept for a tree's normals, timed on a launch with few runs at work, is not the one of all particles'."""
+    xyz, r = synth.crown_splash(pool_layers=6, n_drops=20000)
+    ctx = gpu_context(xyz, r)
+    was = ctx.L.pisurf_run_tuning(1, 1)
+    assert was == 0
+    ctx.build_tree()
+    kept = ctx.L.pisurf_run_tuning(-1, 0)
+    ctx.particle_normals()
+    assert ctx.L.pisurf_run_tuning(-1, 0) == kept + 1
+    ctx.particle_normals()
+    assert ctx.L.pisurf_run_tuning(-1, 0) == kept + 1
+    ctx.close()
