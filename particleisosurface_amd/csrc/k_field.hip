@@ -104,17 +104,25 @@ void launch_eval_points(int prec, GridDev g, const void* ra, const void* rg, Fie
                         double* f, double* grad, Counters* ctr, hipStream_t s) {
     if (n <= 0) return;
     const int m = point_share(n, points_per_wave(prec == 2, grad != nullptr));
-    const unsigned nb = (unsigned)((n + 4 * m - 1) / (4 * m));
+    // 8 or 16 threads a point, and a launch holds fewer than 2^32: slices of 2^27 points (a multiple of a workgroup's 4 m)
+    constexpr int64_t kSlice = int64_t(1) << 27;
     auto go = [&](auto gr, auto mode) {
         constexpr bool G = decltype(gr)::value;
         constexpr int M = decltype(mode)::value;
-        if (prec == 2) {
-            Recs<double> r{(const double4*)ra, (const double4*)rg};
-            k_eval_points<double, false, G, M><<<nb, 256, 0, s>>>(g, r, fc, q, n, m, f, grad, ctr);
-        } else {
-            Recs<float> r{(const float4*)ra, (const float4*)rg};
-            if (prec == 1) k_eval_points<float, true, G, M><<<nb, 256, 0, s>>>(g, r, fc, q, n, m, f, grad, ctr);
-            else k_eval_points<float, false, G, M><<<nb, 256, 0, s>>>(g, r, fc, q, n, m, f, grad, ctr);
+        for (int64_t i = 0; i < n; i += kSlice) {
+            const int64_t k = std::min(kSlice, n - i);
+            const unsigned nb = (unsigned)((k + 4 * m - 1) / (4 * m));
+            const float* qi = q + 3 * i;
+            double* fi = f + i;
+            double* gi = grad ? grad + 3 * i : nullptr;
+            if (prec == 2) {
+                Recs<double> r{(const double4*)ra, (const double4*)rg};
+                k_eval_points<double, false, G, M><<<nb, 256, 0, s>>>(g, r, fc, qi, k, m, fi, gi, ctr);
+            } else {
+                Recs<float> r{(const float4*)ra, (const float4*)rg};
+                if (prec == 1) k_eval_points<float, true, G, M><<<nb, 256, 0, s>>>(g, r, fc, qi, k, m, fi, gi, ctr);
+                else k_eval_points<float, false, G, M><<<nb, 256, 0, s>>>(g, r, fc, qi, k, m, fi, gi, ctr);
+            }
         }
     };
     point_dispatch(field_mode(fc), [&](auto mode) {
