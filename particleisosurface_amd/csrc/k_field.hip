@@ -342,8 +342,9 @@ void launch_uniform_grid(int prec, GridDev g, const void* ra, const void* rg, Fi
         lb.n[a] = (ub.dims[a] + lb.shift[a] + width - 1) / width;
         blocks *= lb.n[a];
     }
-    // (cells of another size: 64 points in more than 16 cells share too little)
-    const bool waves = per_cell >= kWaveDensity && blocks <= INT32_MAX;
+    // (cells of another size: 64 points in more than 16 cells share too little; a sheet fills as little as a third
+    // of its blocks, and a launch holds fewer than 2^32 threads)
+    const bool waves = per_cell >= kWaveDensity && blocks < (1 << 24);
     const unsigned nb = (unsigned)((total + 255) / 256);
     auto go = [&](auto mode) {
         constexpr int M = decltype(mode)::value;
