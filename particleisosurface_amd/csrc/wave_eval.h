@@ -226,7 +226,8 @@ __device__ __forceinline__ int wave_visit(const GridDev& g, const Pol& pol, type
                 pol.stage(L.rec, t, c - d, a);
                 const float x = float(a[0] - Real(ox)) * ic, y = float(a[1] - Real(oy)) * ic,
                             z = float(a[2] - Real(oz)) * ic;
-                const float a2 = x * x + y * y + z * z, r2 = float(a[3]) * ic * ic;
+                // (in cells before it is narrowed: a small radius' square is no normal float)
+                const float a2 = x * x + y * y + z * z, r2 = float(a[3] * Real(ic) * Real(ic));
                 const float w = a2 - r2 - kWaveSlack * (a2 + r2);
                 // a NaN or unbounded record always passes: it reaches every sum of its window
                 const bool fin = fabsf(w) < 1e30f;
