@@ -287,13 +287,19 @@ struct Transfer {
         if (e != hipSuccess) fail(e);
         for (int i = 0; i < k; i++) issued[(p + i) % nb].store((p + i) / nb + 1, std::memory_order_release);
     }
+    // the i-th look at a flag in vain: the link fills a chunk in 0.6 us; what takes longer than some 4096 looks is a
+    // kernel before the copy, or a thread that wants this processor
+    static void relax(uint32_t i) {
+        if (i < 4096) __builtin_ia32_pause();
+        else sched_yield();
+    }
     // chunk c of piece p has been copied by the device
     bool wait_chunk(int p, size_t c) {
         const int b = p % nb;
         const uint32_t want = base[b] + 1 + p / nb;
         volatile uint32_t* w = blk[b]->flag(c);
         for (uint32_t i = 1; *w != want; i++) {
-            __builtin_ia32_pause();
+            relax(i);
             if ((i & 4095) == 0) {
                 if (!ok()) return false;
                 if (issued[b].load(std::memory_order_acquire) <= p / nb) continue;
@@ -337,9 +343,9 @@ struct Transfer {
             }
         } else {
             if (p >= nb) {
-                while (issued[b].load(std::memory_order_acquire) < p / nb) {
+                for (uint32_t i = 1; issued[b].load(std::memory_order_acquire) < p / nb; i++) {
                     if (!ok()) return;
-                    __builtin_ia32_pause();
+                    relax(i);
                 }
                 if (!wait_piece(p - nb)) return;
             }
@@ -423,6 +429,9 @@ hipError_t staged_copy(void* dst, const void* src, size_t bytes, bool down, int 
             t.left[p].store(k, std::memory_order_relaxed);
             t.launch(p, k);
         }
+    // Kernels queued before the copy may run for long: the caller waits for them alone, and the workers, which other
+    // callers share, are woken when data flows.
+    if (down && t.pieces > 1) (void)t.wait_chunk(0, 0);
     host_parallel(t.pieces, t);
     if (!down)
         for (int p = std::max(0, t.pieces - t.nb); p < t.pieces && t.ok(); p++) (void)t.wait_piece(p);
