@@ -4,9 +4,10 @@
 // pages for the length of the call: 16 GB/s down, 28 GB/s up, and 400 - 900 us for 1 - 2 MB, where the link
 // moves 53 GB/s. Here the bytes pass through page-locked blocks. A kernel copies between a block and device
 // memory and flags each 32 KB chunk in host memory when its copy is complete, so neither copies nor
-// reuse of a block need an event or a call into the runtime; the caller's thread and up to 7 workers copy
-// between blocks and the caller's memory, and take the page faults of a fresh array, while the link moves the
-// next group of blocks.
+// reuse of a block need an event or a call into the runtime; the caller's thread and up to 7 workers (one fewer than it
+// has processors at most) copy between blocks and the caller's memory, and take the page faults of a fresh array,
+// while the link moves the next group of blocks. Before a download the workers sleep until its first chunk is there:
+// polling through the kernels before it, they took 52 ms of processor time for a 10 ms kernel, now 10.5.
 //
 // Microseconds (runtime's copy -> this one), arrays touched before: down 1 MB 440 -> 62, 2 MB 870 -> 110, 8 MB
 // 485 -> 250, 24 MB 1500 -> 640; up 1 MB 390 -> 55, 2 MB 740 -> 100, 8 MB 320 -> 300, 24 MB 850 -> 730. A thread

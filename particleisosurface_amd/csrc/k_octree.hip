@@ -988,8 +988,8 @@ __global__ void __launch_bounds__(256) k_classify(GridDev g, Recs<R> rec, FieldC
                         vz = pc[2];
                     }
                     qefs++;
-                    // the field at the vertex is summed by k_qef_values (fewer registers than the
-                    // solve needs); until then the value slot says whether the DMC error zeroes it
+                    // the field at the vertex is summed by k_wave_qef_values or k_point_qef_values (fewer
+                    // registers than the solve needs); until then the value slot says whether the DMC error zeroes it
                     fval = (err / R(__fmul_rn(2.0f, c.w)) < R(0.0001)) ? R(0) : R(1);
                 } else {
                     float p13[3];
@@ -1347,7 +1347,6 @@ static void launch_run_samples(int prec, int T, GridDev g, const void* ra, const
     else m1 ? go(std::integral_constant<int, 128>(), M1()) : go(std::integral_constant<int, 128>(), M0());
 }
 
-// one launch of the sample waves
 // Levels of 8 and more points per hash cell are merged per tile and, from kWaveNodes nodes on (about 70 k points),
 // evaluated 64 to a wave; fewer, by a wave per few points, as such a launch lasts as long as its slowest wave (three
 // levels of a 14 k-particle frame, 7834 nodes the last: 0.12 ms with that one as waves, 0.15 ms without). At 1

@@ -30,8 +30,9 @@ struct RunShape {
 // built (leaf centres: from kWaveMin on). The octree's levels hold 64 or more (deepest sampled, leaf centres), 8 and 1
 // points per cell, level by level upwards. At 64 and 8 a wave's points share a few cells, so one test of all of
 // them against the union of their windows beats each thread testing its own window: crown splash, 4 M
-// particles, compensated FP32, 11.9 M + 2.4 M points: 1.65 ms against 2.05 ms as runs, centres 0.46 against
-// 0.57 ms. At 1 a wave spans five row pieces and tests 18 candidates for each one in a point's
+// particles, compensated FP32, both levels' 11.9 M + 2.4 M distinct points sorted over the level: 1.65 ms against
+// 2.05 ms as runs (samples come by tiles now, without the sort and its merging: both levels 2.19 ms); centres,
+// which are sorted, 0.46 against 0.57 ms. At 1 a wave spans five row pieces and tests 18 candidates for each one in a point's
 // window: 0.70 ms against 0.52 ms for D_min's 1.05 M points.
 constexpr double kWaveDensity = 4.0;
 constexpr int64_t kWaveMin = 1 << 18;

@@ -18,8 +18,9 @@
 //    and wave gathers the sign bits;
 //  - each lane walks its own pass bits over the whole chunk, so a wave takes as many steps as its busiest point has
 //    passing candidates in the chunk (52 at the crown splash's deepest level; word by word it is 70).
-// Deepest level of the crown splash (11.9 M points sorted over the level): 1.20 ms, 60 vector instructions per point,
-// against 1.5 ms and 90.
+// Deepest sampled level of the crown splash, its 11.9 M distinct points sorted by cell over the level (as leaf centres and a
+// caller's many points come): 1.20 ms, 60 vector instructions per point, against 1.5 ms and 90 as runs. Its 14.7 M
+// records as the tiles of nodes list them, without that sort: 1.5 ms.
 // A chunk of 224 candidates takes a tenth fewer instructions, but its LDS leaves two waves per SIMD instead of
 // four, and the kernel 1.5 times as long. Sorting the points by their passing candidates before dealing them to
 // the lanes saves a tenth of the instructions (two points per lane) and loses as much to the occupancy.
@@ -214,7 +215,7 @@ __device__ __forceinline__ int wave_visit(const GridDev& g, const Pol& pol, type
         pt.set(float(q[0] - Real(ox)) * ic, float(q[1] - Real(oy)) * ic, float(q[2] - Real(oz)) * ic);
         for (int cb = 0; cb < total; cb += Pol::kChunk) {
             const int n = min((int)Pol::kChunk, total - cb);
-            // batches of 64 nb slots, words of wl
+            // batches of 16 nb slots, four words of wl = 4 nb each
             const int nbatch = (n + kWaveBatch - 1) / kWaveBatch;
             const int nb = (n + 16 * nbatch - 1) / (16 * nbatch), wl = 4 * nb;
             for (int t = lane; t < n; t += kWave) {
